@@ -36,22 +36,37 @@ DEVI const float *aux_input(const PmlFace &f, int istage) {
   return istage == 0 ? f.pre : (istage == 1 ? f.la : (istage == 2 ? f.lb : f.lc));
 }
 
-/* av: the stage input's values at slab point ia (already read), ar: the
-   auxiliary rhs */
-DEVI void aux_update(const PmlFace &f, const VolArgs &a, long poff, long ia, const float *av, const float *ar) {
+/* byte offset of (i, j, k) in one component of the face's arrays, which are
+   smaller than a field */
+DEVI unsigned face_off(const PmlFace &f, int i, int j, int k) {
+  return (unsigned)(((k - f.k1) * f.bn + (j - f.j1)) * f.an + (i - f.ax0)) * 4u;
+}
+
+/* components C0 .. C0+NC-1 at byte offset oa; av: the stage input's values
+   there (already read), ar: the auxiliary rhs */
+template <int C0, int NC>
+DEVI void aux_update(const PmlFace &f, const VolArgs &a, long poff, unsigned oa, const float *av, const float *ar) {
+  poff += C0 * f.n;
   const float *pre = f.pre + poff;
+  float pv[NC];
   if (a.istage < 3) {
     float *out = (a.istage == 0 ? f.la : (a.istage == 1 ? f.lb : f.lc)) + poff;
 #pragma unroll
-    for (int c = 0; c < 9; c++) out[c * f.n + ia] = (a.istage == 0 ? av[c] : pre[c * f.n + ia]) + a.ca * ar[c];
+    for (int c = 0; c < NC; c++) pv[c] = a.istage == 0 ? av[c] : ld32(pre + c * f.n, oa);
+#pragma unroll
+    for (int c = 0; c < NC; c++) st32(out + c * f.n, oa, pv[c] + a.ca * ar[c]);
   } else {
     float *la = f.la + poff;
     const float *lb = f.lb + poff;
+    float ev[NC], bv[NC];
 #pragma unroll
-    for (int c = 0; c < 9; c++) {
-      const long q = c * f.n + ia;
-      la[q] = rk_end(pre[q], la[q], lb[q], av[c], a.cb * ar[c]);
+    for (int c = 0; c < NC; c++) {
+      pv[c] = ld32(pre + c * f.n, oa);
+      ev[c] = ld32(la + c * f.n, oa);
+      bv[c] = ld32(lb + c * f.n, oa);
     }
+#pragma unroll
+    for (int c = 0; c < NC; c++) st32(la + c * f.n, oa, rk_end(pv[c], ev[c], bv[c], av[c], a.cb * ar[c]));
   }
 }
 
@@ -67,7 +82,7 @@ DEVI void pml_point(const VolArgs &a, int i, int j, int k, long p, const float *
       const PmlFace &f = a.pml[dim][side];
       if (!f.on) continue;
       if (i < f.i1 || i > f.i2 || j < f.j1 || j > f.j2 || k < f.k1 || k > f.k2) continue;
-      long ia = (long)(k - f.k1) * ((long)f.bn * f.an) + (long)(j - f.j1) * f.an + (i - f.ax0);
+      const unsigned oa = face_off(f, i, j, k);
       int ic = dim == 0 ? i - f.i1 : (dim == 1 ? j - f.j1 : k - f.k1);
       float cD = f.D[ic], cA = f.A[ic], cB = f.B[ic];
       float cB1 = cB - 1.0f;
@@ -88,7 +103,7 @@ DEVI void pml_point(const VolArgs &a, int i, int j, int k, long p, const float *
       const float *auxc = aux_input(f, a.istage) + poff;
       float av[9], ar[9];
 #pragma unroll
-      for (int c = 0; c < 9; c++) av[c] = auxc[c * f.n + ia];
+      for (int c = 0; c < 9; c++) av[c] = ld32(auxc + c * f.n, oa);
 #pragma unroll
       for (int c = 0; c < 9; c++) {
         h[c] += cB1 * r[c] - cB * av[c];
@@ -116,7 +131,7 @@ DEVI void pml_point(const VolArgs &a, int i, int j, int k, long p, const float *
         }
       }
       /* auxiliary RK update; the slab point is owned by this thread only */
-      aux_update(f, a, poff, ia, av, ar);
+      aux_update<0, 9>(f, a, poff, oa, av, ar);
     }
   }
 }
@@ -132,42 +147,72 @@ DEVI bool fault_column(const FaultSkip &fs, int i, long pf) {
 
 /* RK stage update of the nine wavefield components at p: stages 0..2 write
    the next stage input pre + a_s dt h (wav_update, wav_t.cu:218-226),
-   stage 3 the level at t_{n+1} over level A (rk_end) */
+   stage 3 the level at t_{n+1} over level A (rk_end). Every load stands
+   before the first store: the compiler may not move a load over a store that
+   could alias it, and a load, store, load, ... sequence waits for memory once
+   per component (grouped, the top-layer kernel takes 0.034 ms per stage
+   instead of 0.047 at 160 x 240 x 100) */
 DEVI void rk_point(const VolArgs &a, long p, const float *h, long woff = 0) {
   const long sc = a.g.sicmp;
   p += woff;
   if (a.istage < 3) {
+    float pv[9];
 #pragma unroll
-    for (int c = 0; c < 9; c++) a.tnew[c * sc + p] = a.pre[c * sc + p] + a.ca * h[c];
+    for (int c = 0; c < 9; c++) pv[c] = a.pre[c * sc + p];
+#pragma unroll
+    for (int c = 0; c < 9; c++) a.tnew[c * sc + p] = pv[c] + a.ca * h[c];
   } else {
+    float pv[9], ev[9], bv[9], cv[9];
 #pragma unroll
     for (int c = 0; c < 9; c++) {
-      const long q = c * sc + p;
-      a.end[q] = rk_end(a.pre[q], a.end[q], a.lb[q], a.cur[q], a.cb * h[c]);
+      pv[c] = a.pre[c * sc + p];
+      ev[c] = a.end[c * sc + p];
+      bv[c] = a.lb[c * sc + p];
+      cv[c] = a.cur[c * sc + p];
     }
+#pragma unroll
+    for (int c = 0; c < 9; c++) a.end[c * sc + p] = rk_end(pv[c], ev[c], bv[c], cv[c], a.cb * h[c]);
   }
 }
 
-/* rk_point with 32-bit byte offsets (o = 4 p) from the scenario's levels;
-   the stage input's own value at stage 3 comes from the cache (the stencil
-   has just read it) */
-DEVI void rk_point32(const VolArgs &a, unsigned o, const float *h, long woff = 0) {
+/* rk_point with 32-bit byte offsets (o = 4 p) from the scenario's levels,
+   for components C0 .. C0+NC-1; the stage input's own value at stage 3 comes
+   from the cache (the stencil has just read it). Loads first, as in
+   rk_point. */
+template <int C0, int NC>
+DEVI void rk_part32(const VolArgs &a, unsigned o, const float *h, long woff) {
   const long sc = a.g.sicmp;
+  woff += C0 * sc;
   const float *pre = a.pre + woff;
+  float pv[NC];
+#pragma unroll
+  for (int c = 0; c < NC; c++) pv[c] = ld32nt(pre + c * sc, o);
   if (a.istage < 3) {
     float *tnew = a.tnew + woff;
 #pragma unroll
-    for (int c = 0; c < 9; c++) st32nt(tnew + c * sc, o, ld32nt(pre + c * sc, o) + a.ca * h[c]);
+    for (int c = 0; c < NC; c++) st32nt(tnew + c * sc, o, pv[c] + a.ca * h[c]);
   } else {
     float *end = a.end + woff;
     const float *lb = a.lb + woff, *cur = a.cur + woff;
+    float ev[NC], bv[NC], cv[NC];
 #pragma unroll
-    for (int c = 0; c < 9; c++) {
-      const float v = rk_end(ld32nt(pre + c * sc, o), ld32nt(end + c * sc, o), ld32nt(lb + c * sc, o),
-                             ld32(cur + c * sc, o), a.cb * h[c]);
-      st32nt(end + c * sc, o, v);
+    for (int c = 0; c < NC; c++) {
+      ev[c] = ld32nt(end + c * sc, o);
+      bv[c] = ld32nt(lb + c * sc, o);
+      cv[c] = ld32(cur + c * sc, o);
     }
+#pragma unroll
+    for (int c = 0; c < NC; c++) st32nt(end + c * sc, o, rk_end(pv[c], ev[c], bv[c], cv[c], a.cb * h[c]));
   }
+}
+/* in groups of three components: with all nine in flight the interior kernel
+   takes 61 VGPRs instead of 43 and 1% longer at 400 x 800 x 266, one by one
+   it is 1% faster there and 10-15% slower up to 160 x 240 x 100 (0.094 ->
+   0.086 ms per stage) */
+DEVI void rk_point32(const VolArgs &a, unsigned o, const float *h, long woff = 0) {
+  rk_part32<0, 3>(a, o, h, woff);
+  rk_part32<3, 3>(a, o, h + 3, woff);
+  rk_part32<6, 3>(a, o, h + 6, woff);
 }
 
 /* rhs + PML + RK update of one point from its 27 derivatives */

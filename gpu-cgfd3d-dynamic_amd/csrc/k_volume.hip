@@ -243,11 +243,19 @@ __global__ void __launch_bounds__(256, 8) k_vol_acc_slab(VolArgs a, BatArgs b) {
  * Lean CFS-PML point. The correction of face `dim` needs the part of every
  * rhs component that comes from the derivatives along `dim` only (r below;
  * the r[] of sv_curv_col_el_iso_gpu.cu:916-1288). Those parts are
- * accumulated field by field, like the interior kernel's gradient sums, with
- * a register fence per field, so only 27 partial sums, the metric and the
- * media stay live; the full rhs is their sum over the three directions.
- * Then each face containing the point applies its correction and advances
- * its auxiliary variables in the reference's face order. The free-surface
+ * accumulated field by field, like the interior kernel's gradient sums; the
+ * full rhs is their sum over the three directions. Then each face containing
+ * the point applies its correction and advances its auxiliary variables in
+ * the reference's face order. The velocity rhs uses the stress fields alone
+ * and the stress rhs the velocity alone, so a point is done in two phases,
+ * velocity first, each through to its stores: 9 and then 18 partial sums are
+ * live instead of 27. What bounds a band point is the number of times its
+ * wave waits for memory, so a phase has three fields' taps in flight at once
+ * and loads a face's auxiliaries, and then the RK levels, in groups ahead of
+ * their stores, at 5 waves per SIMD (93 VGPRs, no spills). Per stage against
+ * the 27-sum form with a fence per field at 7 waves per SIMD (72 VGPRs, 8-24
+ * bytes of spills): 0.481 -> 0.447 ms at 200 x 400 x 150, 1.97 -> 1.88 ms at
+ * 400 x 800 x 266, 0.050 -> 0.040 ms at 80 x 120 x 60. The free-surface
  * term of the x/y faces (k == nk2) never occurs here: with a free surface
  * the top four layers belong to k_vol_top.
  * ---------------------------------------------------------------------- */
@@ -273,72 +281,80 @@ DEVI constexpr int pml_slot(int d) {
   return ((DM >> d) & 1) ? s : pml_nslot<DM>() - 1;
 }
 
-template <bool VC, int DM, class Deriv>
-DEVI void pml_core(const VolArgs &a, const BatArgs &b, int i, int j, int k, int sn, Deriv deriv) {
-  constexpr int NS = pml_nslot<DM>();
-  const long sc = a.g.sicmp, sy = a.g.siy, sz = a.g.siz;
-  const long p = i + j * sy + (long)k * sz;
-  const unsigned o = (unsigned)p * 4u;
-  const float *M = a.met;
-  const long woff = (long)sn * b.wstride;
-  float e[3][3];  /* rows: xi, eta, zeta derivatives (x, y, z components) */
-#pragma unroll
-  for (int d = 0; d < 3; d++)
-#pragma unroll
-    for (int c = 0; c < 3; c++) e[d][c] = met_zero<VC>(d, c) ? 0.0f : ld32nt(M + (1 + 3 * d + c) * sc, o);
-  const float l = ld32nt(a.lam, o), m = ld32nt(a.mu, o), s = ld32nt(a.slw, o);
-  const float l2m = l + 2.0f * m;
-  float r[NS][9];
+/* does the derivative of field f along d enter the rhs */
+template <bool VC>
+DEVI constexpr bool deriv_used(int f, int d) { return !VC || d == 2 || grad_used(f, d); }
+
+/* what the derivative D of field f along d adds to the velocity rhs (PH 0:
+   f a stress, r[0..2]) or the stress rhs (PH 1: f a velocity, r[0..5] =
+   Txx .. Txy), with row d of the metric e */
+template <bool VC, int PH>
+DEVI void add_part(int f, int d, float D, const float *e, float l, float m, float l2m, float s, float *r) {
+  const bool n1 = !met_zero<VC>(d, 0), n2 = !met_zero<VC>(d, 1), n3 = !met_zero<VC>(d, 2);
+  const float e1 = e[0], e2 = e[1], e3 = e[2];
+  if (PH == 0) {
+    switch (f) {
+      case TXX: if (n1) r[VX] += s * e1 * D; break;
+      case TYY: if (n2) r[VY] += s * e2 * D; break;
+      case TZZ: if (n3) r[VZ] += s * e3 * D; break;
+      case TXY: if (n2) r[VX] += s * e2 * D; if (n1) r[VY] += s * e1 * D; break;
+      case TXZ: if (n3) r[VX] += s * e3 * D; if (n1) r[VZ] += s * e1 * D; break;
+      case TYZ: if (n3) r[VY] += s * e3 * D; if (n2) r[VZ] += s * e2 * D; break;
+    }
+    return;
+  }
+  switch (f) {
+    case VX:
+      if (n1) { r[TXX - 3] += l2m * e1 * D; r[TYY - 3] += l * e1 * D; r[TZZ - 3] += l * e1 * D; }
+      if (n2) r[TXY - 3] += m * e2 * D;
+      if (n3) r[TXZ - 3] += m * e3 * D;
+      break;
+    case VY:
+      if (n2) { r[TXX - 3] += l * e2 * D; r[TYY - 3] += l2m * e2 * D; r[TZZ - 3] += l * e2 * D; }
+      if (n1) r[TXY - 3] += m * e1 * D;
+      if (n3) r[TYZ - 3] += m * e3 * D;
+      break;
+    case VZ:
+      if (n3) { r[TXX - 3] += l * e3 * D; r[TYY - 3] += l * e3 * D; r[TZZ - 3] += l2m * e3 * D; }
+      if (n1) r[TXZ - 3] += m * e1 * D;
+      if (n2) r[TYZ - 3] += m * e2 * D;
+      break;
+  }
+}
+
+/* One phase of a CFS-PML point: PH 0 the velocity components, 1 the stress
+   components. own: the point's RK update belongs to the volume kernels. */
+template <bool VC, int DM, int PH, class Deriv>
+DEVI void pml_phase(const VolArgs &a, int i, int j, int k, unsigned o, long woff, long poff, const float (&e)[3][3],
+                    float l, float m, float l2m, float s, bool own, Deriv deriv) {
+  constexpr int NS = pml_nslot<DM>(), C0 = PH == 0 ? 0 : 3, NC = PH == 0 ? 3 : 6;
+  constexpr int F0 = PH == 0 ? 3 : 0, F1 = PH == 0 ? 9 : 3;
+  const long sc = a.g.sicmp;
+  float r[NS][NC];
 #pragma unroll
   for (int d = 0; d < NS; d++)
 #pragma unroll
-    for (int c = 0; c < 9; c++) r[d][c] = 0.0f;
+    for (int c = 0; c < NC; c++) r[d][c] = 0.0f;
 #pragma unroll
-  for (int f = 0; f < 9; f++) {
-    float D0, D1, D2;
-    deriv(f, o, D0, D1, D2);
-    if (!VC || grad_used(f, 0)) __asm__ volatile("" : "+v"(D0));
-    if (!VC || grad_used(f, 1)) __asm__ volatile("" : "+v"(D1));
-    __asm__ volatile("" : "+v"(D2) : : "memory");
-#pragma unroll
-    for (int d = 0; d < 3; d++) {
-      const float Dd = d == 0 ? D0 : (d == 1 ? D1 : D2);
-      const float e1 = e[d][0], e2 = e[d][1], e3 = e[d][2];
-      const bool n1 = !met_zero<VC>(d, 0), n2 = !met_zero<VC>(d, 1), n3 = !met_zero<VC>(d, 2);
-      float *const rd = r[pml_slot<DM>(d)];
-      switch (f) {
-        case TXX: if (n1) rd[VX] += s * e1 * Dd; break;
-        case TYY: if (n2) rd[VY] += s * e2 * Dd; break;
-        case TZZ: if (n3) rd[VZ] += s * e3 * Dd; break;
-        case TXY: if (n2) rd[VX] += s * e2 * Dd; if (n1) rd[VY] += s * e1 * Dd; break;
-        case TXZ: if (n3) rd[VX] += s * e3 * Dd; if (n1) rd[VZ] += s * e1 * Dd; break;
-        case TYZ: if (n3) rd[VY] += s * e3 * Dd; if (n2) rd[VZ] += s * e2 * Dd; break;
-        case VX:
-          if (n1) { rd[TXX] += l2m * e1 * Dd; rd[TYY] += l * e1 * Dd; rd[TZZ] += l * e1 * Dd; }
-          if (n2) rd[TXY] += m * e2 * Dd;
-          if (n3) rd[TXZ] += m * e3 * Dd;
-          break;
-        case VY:
-          if (n2) { rd[TXX] += l * e2 * Dd; rd[TYY] += l2m * e2 * Dd; rd[TZZ] += l * e2 * Dd; }
-          if (n1) rd[TXY] += m * e1 * Dd;
-          if (n3) rd[TYZ] += m * e3 * Dd;
-          break;
-        case VZ:
-          if (n3) { rd[TXX] += l * e3 * Dd; rd[TYY] += l * e3 * Dd; rd[TZZ] += l2m * e3 * Dd; }
-          if (n1) rd[TXZ] += m * e1 * Dd;
-          if (n2) rd[TYZ] += m * e2 * Dd;
-          break;
-      }
+  for (int f = F0; f < F1; f++) {
+    float D[3];
+    deriv(f, o, D[0], D[1], D[2]);
+    if ((f - F0) % 3 == 2) {  /* three fields' taps in flight at a time */
+      if (deriv_used<VC>(f, 0)) __asm__ volatile("" : "+v"(D[0]));
+      if (deriv_used<VC>(f, 1)) __asm__ volatile("" : "+v"(D[1]));
+      __asm__ volatile("" : "+v"(D[2]) : : "memory");
     }
-  }
-  float h[9];
 #pragma unroll
-  for (int c = 0; c < 9; c++) {
+    for (int d = 0; d < 3; d++)
+      if (deriv_used<VC>(f, d)) add_part<VC, PH>(f, d, D[d], e[d], l, m, l2m, s, r[pml_slot<DM>(d)]);
+  }
+  float h[NC];
+#pragma unroll
+  for (int c = 0; c < NC; c++) {
     h[c] = r[0][c];
 #pragma unroll
     for (int q = 1; q < NS; q++) h[c] += r[q][c];
   }
-  const long poff = (long)sn * b.pstride;
 #pragma unroll
   for (int dim = 0; dim < 3; dim++) {
     if (!((DM >> dim) & 1)) continue;
@@ -348,23 +364,44 @@ DEVI void pml_core(const VolArgs &a, const BatArgs &b, int i, int j, int k, int 
       const PmlFace &F = a.pml[dim][side];
       if (!F.on) continue;
       if (i < F.i1 || i > F.i2 || j < F.j1 || j > F.j2 || k < F.k1 || k > F.k2) continue;
-      const long ia = (long)(k - F.k1) * ((long)F.bn * F.an) + (long)(j - F.j1) * F.an + (i - F.ax0);
-      const int ic = dim == 0 ? i - F.i1 : (dim == 1 ? j - F.j1 : k - F.k1);
-      const float cD = F.D[ic], cA = F.A[ic], cB = F.B[ic];
+      const unsigned oa = face_off(F, i, j, k);
+      const unsigned ic = (unsigned)(dim == 0 ? i - F.i1 : (dim == 1 ? j - F.j1 : k - F.k1)) * 4u;
+      const float cD = ld32(F.D, ic), cA = ld32(F.A, ic), cB = ld32(F.B, ic);
       const float cB1 = cB - 1.0f;
-      const float *auxc = aux_input(F, a.istage) + poff;
-      float av[9], ar[9];
+      const float *auxc = aux_input(F, a.istage) + poff + C0 * F.n;
+      float av[NC], ar[NC];
 #pragma unroll
-      for (int c = 0; c < 9; c++) {
-        av[c] = auxc[c * F.n + ia];
+      for (int c = 0; c < NC; c++) av[c] = ld32(auxc + c * F.n, oa);
+#pragma unroll
+      for (int c = 0; c < NC; c++) {
         h[c] += cB1 * rdim[c] - cB * av[c];
         ar[c] = cD * rdim[c] - cA * av[c];
       }
-      aux_update(F, a, poff, ia, av, ar);
+      aux_update<C0, NC>(F, a, poff, oa, av, ar);
     }
   }
-  if (a.fs.nfault > 0 && fault_column(a.fs, i, j + (long)k * a.g.ny)) return;
-  rk_point32(a, o, h, woff);
+  if (own) rk_part32<C0, NC>(a, o, h, woff);
+}
+
+template <bool VC, int DM, class Deriv>
+DEVI void pml_core(const VolArgs &a, const BatArgs &b, int i, int j, int k, int sn, Deriv deriv) {
+  const long sc = a.g.sicmp, sy = a.g.siy, sz = a.g.siz;
+  const long p = i + j * sy + (long)k * sz;
+  const unsigned o = (unsigned)p * 4u;
+  const float *M = a.met;
+  const long woff = (long)sn * b.wstride, poff = (long)sn * b.pstride;
+  float e[3][3];  /* rows: xi, eta, zeta derivatives (x, y, z components) */
+#pragma unroll
+  for (int d = 0; d < 3; d++)
+#pragma unroll
+    for (int c = 0; c < 3; c++) e[d][c] = met_zero<VC>(d, c) ? 0.0f : ld32nt(M + (1 + 3 * d + c) * sc, o);
+  const float l = ld32nt(a.lam, o), m = ld32nt(a.mu, o), s = ld32nt(a.slw, o);
+  const float l2m = l + 2.0f * m;
+  const bool own = !(a.fs.nfault > 0 && fault_column(a.fs, i, j + (long)k * a.g.ny));
+  pml_phase<VC, DM, 0>(a, i, j, k, o, woff, poff, e, l, m, l2m, s, own, deriv);
+  /* the second phase's loads stay below the first one's stores */
+  __asm__ volatile("" : : : "memory");
+  pml_phase<VC, DM, 1>(a, i, j, k, o, woff, poff, e, l, m, l2m, s, own, deriv);
 }
 
 template <int ID, int JD, int KD, bool VC = false, int DM = 7>
@@ -380,10 +417,8 @@ DEVI void pml_acc_point(const VolArgs &a, const BatArgs &b, int i, int j, int k,
   });
 }
 
-/* at least 6 waves per SIMD: 71 VGPRs without spills (the compiler's own
-   choice, 87 VGPRs, leaves 5 waves and runs the PML tiles 13% slower) */
 template <int ID, int JD, int KD>
-__global__ void __launch_bounds__(256, 6) k_vol_pml_lean(VolArgs a, BatArgs b) {
+__global__ void __launch_bounds__(256, 5) k_vol_pml_lean(VolArgs a, BatArgs b) {
   const int k = a.k_lo + (int)blockIdx.z + 3;
   const int bi0 = blockIdx.x * 64, bj0 = blockIdx.y * 4 + 3;
   if (!block_touches_pml(a, bi0, bi0 + 63, bj0, bj0 + 3, k)) return;
@@ -445,11 +480,8 @@ DEVI bool band_point(const VolBands &r, long L0, int &i, int &j, int &k) {
   return by < r.nty[q] && i >= r.x0[q] && i < r.x1[q] && j < r.y1[q];
 }
 
-/* 7 waves per SIMD: 72 VGPRs and 8-24 bytes of spills per lane; 1.3% faster
-   than the 6 waves the compiler picks without the bound (75 VGPRs), while
-   8 waves (64 VGPRs, 40-56 bytes of spills) lose it again */
 template <int ID, int JD, int KD, bool VC, int DM>
-__global__ void __launch_bounds__(256, 7) k_vol_pml_band(VolArgs a, BatArgs b, VolBands r) {
+__global__ void __launch_bounds__(256, 5) k_vol_pml_band(VolArgs a, BatArgs b, VolBands r) {
   int i, j, k;
   if (!band_point(r, blockIdx.x, i, j, k)) return;
   pml_acc_point<ID, JD, KD, VC, DM>(a, b, i, j, k, b.act[0]);
@@ -500,7 +532,7 @@ __global__ void __launch_bounds__(256, 8) k_vol_bat_acc_box_slab(VolArgs a, BatA
 }
 
 template <int ID, int JD, int KD, bool VC, int DM>
-__global__ void __launch_bounds__(256, 7) k_vol_bat_pml_band(VolArgs a, BatArgs b, VolBands r) {
+__global__ void __launch_bounds__(256, 5) k_vol_bat_pml_band(VolArgs a, BatArgs b, VolBands r) {
   const long per = r.cum[r.n];
   const int sq = (int)(blockIdx.x / per);
   int i, j, k;
@@ -652,7 +684,7 @@ __global__ void __launch_bounds__(256, 8) k_vol_bat_acc(VolArgs a, BatArgs b, lo
 }
 
 template <int ID, int JD, int KD>
-__global__ void __launch_bounds__(256, 6) k_vol_bat_pml(VolArgs a, BatArgs b, long nitems) {
+__global__ void __launch_bounds__(256, 5) k_vol_bat_pml(VolArgs a, BatArgs b, long nitems) {
   int bx, by, kz, q;
   if (!bat_item(a, b, 1, nitems, bx, by, kz, q)) return;
   const int k = a.k_lo + kz + 3;
