@@ -48,6 +48,71 @@ DEVI void metric_cols_f(const float *fm, long ss, long pf, float M[3][3]) {
   M[2][0] = fm[3 * ss + pf]; M[2][1] = fm[6 * ss + pf]; M[2][2] = fm[9 * ss + pf];
 }
 
+/* ---- operators on loaded taps ----
+   The node kernels are bound by how often a lane waits for memory (a plane
+   is a few thousand lanes, a node some hundred loads), so each kernel loads
+   the taps it may need before it branches on the node's kind, and every load
+   of a phase stands before the phase's first store; blocks are one wavefront,
+   so a small plane spreads over the CUs. Per stage, against loads inside the
+   branches and between the stores: k_fault_nodes 30.3 -> 12.2 us on a 48 x 28
+   plane, 53 -> 20 on 240 x 100, 136 -> 97 on 800 x 266; k_trial 16.2 -> 7.7,
+   22 -> 11, 58 -> 40. The taps of the one-sided
+   five-point operator are v[0..4] = p[o], o = -1..3 (forward, F = 1) or -3..1.
+   The formulas and their term order are those of fd_t.h (macdrp, mac22,
+   mac24); the direction is a template argument because with both forms in one
+   expression the compiler shares their products and fuses others into FMAs. */
+template <int F>
+DEVI void taps5(const float *p, long s, float *v) {
+  const float *q = p - (F == 1 ? s : 3 * s);
+#pragma unroll
+  for (int n = 0; n < 5; n++) v[n] = q[n * s];
+}
+template <int F>
+DEVI float t_drp(const float *v) {
+  return F == 1 ? (float)((kC1 * v[0]) + (kC2 * v[1]) + (kC3 * v[2]) + (kC4 * v[3]) + (kC5 * v[4]))
+                : (float)(-(kC1 * v[4]) - (kC2 * v[3]) - (kC3 * v[2]) - (kC4 * v[1]) - (kC5 * v[0]));
+}
+template <int F>
+DEVI float t_22(const float *v) { return F == 1 ? v[2] - v[1] : v[3] - v[2]; }
+template <int F>
+DEVI float t_24(const float *v) {
+  return F == 1 ? (float)((kB1 * v[1]) + (kB2 * v[2]) + (kB3 * v[3]))
+                : (float)__builtin_fma(-kB3, (double)v[1], __builtin_fma(-kB2, (double)v[2], -kB1 * v[3]));
+}
+/* the value at the node itself */
+template <int F>
+DEVI float t_mid(const float *v) { return F == 1 ? v[1] : v[3]; }
+/* z derivative of a split-node traction with the odd image across the free
+   surface (trial_slipweakening.cu:202-227); n_free = 3..6: the surface's
+   place among the points -3..3. Forward taps of a surface node (n_free = 3)
+   also need the points -3 and -2 (lo). */
+template <int F>
+DEVI float t_free(const float *v, const float *lo, int n_free) {
+  float u[7];
+  if (F == 1) {
+    u[0] = lo[0]; u[1] = lo[1]; u[2] = v[0]; u[3] = v[1]; u[4] = v[2]; u[5] = v[3]; u[6] = v[4];
+  } else {
+    u[0] = v[0]; u[1] = v[1]; u[2] = v[2]; u[3] = v[3]; u[4] = v[4]; u[5] = 0.0f; u[6] = 0.0f;
+  }
+  float w3 = n_free == 3 ? 0.0f : u[3];
+  float w4 = n_free == 3 ? -u[2] : (n_free == 4 ? 0.0f : u[4]);
+  float w5 = n_free == 3 ? -u[1] : (n_free == 4 ? -u[3] : (n_free == 5 ? 0.0f : u[5]));
+  float w6 = n_free == 3 ? -u[0] : (n_free == 4 ? -u[2] : (n_free == 5 ? -u[4] : 0.0f));
+  /* products with a selected constant would be folded and not fused below */
+  __asm__("" : "+v"(w3), "+v"(w4), "+v"(w5), "+v"(w6));
+  return F == 1 ? (float)((kC1 * u[2]) + (kC2 * w3) + (kC3 * w4) + (kC4 * w5) + (kC5 * w6))
+                : (float)(-(kC1 * w4) - (kC2 * w3) - (kC3 * u[2]) - (kC4 * u[1]) - (kC5 * u[0]));
+}
+
+/* jac and the metric at a node, read in the order metric_cols_f reads them */
+DEVI void fault_metric_at(const FaultDev &F, long ss, long pf, float *fm) {
+#pragma unroll
+  for (int r = 0; r < 3; r++)
+#pragma unroll
+    for (int c = 0; c < 3; c++) fm[1 + 3 * c + r] = F.fmet[(1 + 3 * c + r) * ss + pf];
+  fm[0] = F.fmet[pf];
+}
+
 __global__ void __launch_bounds__(256) k_fault_metric(Grid g, const float *__restrict__ met, int i0, float *fmet) {
   const int j = blockIdx.x * 256 + (int)threadIdx.x, k = blockIdx.y;
   if (j >= g.ny) return;
@@ -107,45 +172,38 @@ __global__ void __launch_bounds__(256) k_wave2fault(FaultArgs a, BatArgs b) {
 
 /* split-node average back onto the wavefield column i0 (transform.cu:331-372),
    writing sigma_xz/sigma_yz into swapped arrays unless fix_q1 (the call at
-   transform.cu:274-276 passes Tyz, Txz to parameters named Txz, Tyz) */
-DEVI void fault2wave_node(const FaultArgs &a, const FaultDev &F, long pf, long p, float *w, const float *fl) {
-  const long sc = a.g.sicmp, ss = a.g.sslice;
+   transform.cu:274-276 passes Tyz, Txz to parameters named Txz, Tyz).
+   fm: jac and the metric on the plane's column; t1: the fault traction; v:
+   the split-node state [component][side] */
+DEVI void fault2wave_node(const FaultArgs &a, const float *fm, const float *t1, const float (&v)[9][2], long p,
+                          float *w) {
+  const long sc = a.g.sicmp;
   float M[3][3], Tr[3][3], S[3][3];
-  metric_cols_f(F.fmet, ss, pf, M);
-  float rj = (float)(1.0 / F.fmet[pf]);
+#pragma unroll
+  for (int r = 0; r < 3; r++)
+#pragma unroll
+    for (int c = 0; c < 3; c++) M[r][c] = fm[1 + 3 * c + r];
+  float rj = (float)(1.0 / fm[0]);
 #pragma unroll
   for (int c = 0; c < 3; c++) {
-    Tr[c][0] = F.T1[(long)c * 7 * ss + 3 * ss + pf];
-    Tr[c][1] = (float)((fl[fidx(3 + c, 0, ss) + pf] + fl[fidx(3 + c, 1, ss) + pf]) * 0.5);
-    Tr[c][2] = (float)((fl[fidx(6 + c, 0, ss) + pf] + fl[fidx(6 + c, 1, ss) + pf]) * 0.5);
+    Tr[c][0] = t1[c];
+    Tr[c][1] = (float)((v[3 + c][0] + v[3 + c][1]) * 0.5);
+    Tr[c][2] = (float)((v[6 + c][0] + v[6 + c][1]) * 0.5);
   }
   inv3(M);
   mm33(Tr, M, S);
 #pragma unroll
-  for (int r = 0; r < 3; r++)
-#pragma unroll
-    for (int c = 0; c < 3; c++) S[r][c] *= rj;
-#pragma unroll
-  for (int c = 0; c < 3; c++) w[c * sc + p] = (float)((fl[fidx(c, 0, ss) + pf] + fl[fidx(c, 1, ss) + pf]) * 0.5);
-  w[TXX * sc + p] = S[0][0];
-  w[TYY * sc + p] = S[1][1];
-  w[TZZ * sc + p] = S[2][2];
-  w[TXY * sc + p] = (float)((S[0][1] + S[1][0]) * 0.5);
-  float sxz = (float)((S[0][2] + S[2][0]) * 0.5);
-  float syz = (float)((S[1][2] + S[2][1]) * 0.5);
+  for (int c = 0; c < 3; c++) w[c * sc + p] = (float)((v[c][0] + v[c][1]) * 0.5);
+  w[TXX * sc + p] = S[0][0] * rj;
+  w[TYY * sc + p] = S[1][1] * rj;
+  w[TZZ * sc + p] = S[2][2] * rj;
+  /* (S01 + S10) rj / 2 and so on, the sum of the two products written as the
+     FMA it compiles to, so both callers round alike */
+  w[TXY * sc + p] = (float)(__builtin_fmaf(S[0][1], rj, S[1][0] * rj) * 0.5);
+  float sxz = (float)(__builtin_fmaf(S[0][2], rj, S[2][0] * rj) * 0.5);
+  float syz = (float)(__builtin_fmaf(S[1][2], rj, S[2][1] * rj) * 0.5);
   w[(a.fix_q1 ? TXZ : TYZ) * sc + p] = sxz;
   w[(a.fix_q1 ? TYZ : TXZ) * sc + p] = syz;
-}
-
-/* z-derivative of a split-node traction with the odd image across the free
-   surface (trial_slipweakening.cu:202-227) */
-DEVI float dz_free_image(const float *col, long ny, int n_free, int kdir) {
-  float v[7];
-#pragma unroll
-  for (int l = -3; l <= 3; l++) v[l + 3] = col[l * ny];
-  v[n_free] = 0.0f;
-  for (int l = n_free + 1; l < 7; l++) v[l] = -v[2 * n_free - l];
-  return vecc(v + 3, kdir);
 }
 
 /* ---------------------------------------------------------------------- */
@@ -193,28 +251,30 @@ __global__ void __launch_bounds__(256) k_trial_t1(FaultArgs a, BatArgs b) {
 }
 
 /* ---------------------------------------------------------------------- */
+template <int JD, int KD>
 DEVI void k_trial_body(const FaultArgs &a, int id) {
   const int iy = blockIdx.x * blockDim.x + threadIdx.x;
   const int iz = blockIdx.y * blockDim.y + threadIdx.y;
   if (iy >= a.g.nj || iz >= a.g.nk) return;
   const FaultDev F = fdev(a, id);
-  const long ss = a.g.sslice, sc = a.g.sicmp, ny = a.g.ny;
+  const long ss = a.g.sslice, ny = a.g.ny;
   const long pf = (iy + 3) + (long)(iz + 3) * ny;
-  if (F.united[pf] != 0) return;
-  const int jdir = a.jdir, kdir = a.kdir;
-  const float *met = a.met;
+  const int united = F.united[pf], ry = F.rupy[pf], rz = F.rupz[pf];
+  if (united != 0) return;
   const long row = (long)(iy + 3) * a.g.siy + (long)(iz + 3) * a.g.siz;
   const long p0 = F.i0 + row;
   const float *fc = a.f_cur + (long)id * 18 * ss;
   const float *fp = a.f_pre + (long)id * 18 * ss;
   const int km = a.g.nk - (iz + 1);
   const int n_free = km + 3;
-  const int ry = F.rupy[pf], rz = F.rupz[pf];
 
+  float fm[10];
+  fault_metric_at(F, ss, pf, fm);
   float Mrho[2], R[2][3];
+  float v[9][2];  /* the split-node state of the stage input at the node */
 #pragma unroll
   for (int m = 0; m < 2; m++) {
-    float jac0 = F.fmet[pf];
+    float jac0 = fm[0];
     float rho = F.rho_f[m * ss + pf];
     Mrho[m] = (float)(0.5 * jac0 * rho);
     float t1[3][3];  /* [comp][l-1]: the traction columns k_trial_t1 wrote */
@@ -224,16 +284,32 @@ DEVI void k_trial_body(const FaultArgs &a, int id) {
 #pragma unroll
       for (int c = 0; c < 3; c++) t1[c][l - 1] = F.T1[(long)c * 7 * ss + slot * ss + pf];
     }
+    float y[3][5], z[3][5];
 #pragma unroll
     for (int c = 0; c < 3; c++) {
-      const float *p2 = fc + fidx(3 + c, m, ss) + pf;
-      const float *p3 = fc + fidx(6 + c, m, ss) + pf;
+      taps5<JD>(fc + fidx(3 + c, m, ss) + pf, 1, y[c]);
+      taps5<KD>(fc + fidx(6 + c, m, ss) + pf, ny, z[c]);
+      v[c][m] = fc[fidx(c, m, ss) + pf];
+    }
+    float lo[3][2] = {};
+    if (a.isfree == 1 && km == 0 && KD == 1) {
+#pragma unroll
+      for (int c = 0; c < 3; c++) {
+        const float *p3 = fc + fidx(6 + c, m, ss) + pf;
+        lo[c][0] = p3[-3 * ny];
+        lo[c][1] = p3[-2 * ny];
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+      v[3 + c][m] = t_mid<JD>(y[c]);
+      v[6 + c][m] = t_mid<KD>(z[c]);
       float dy = 0.0f, dz = 0.0f;
-      if (ry == 1) dy = mac22(p2, 1, jdir);
-      if (ry == 0) dy = macdrp(p2, 1, jdir);
-      if (rz == 1) dz = mac22(p3, ny, kdir);
-      if (rz == 0) dz = macdrp(p3, ny, kdir);
-      if (a.isfree == 1 && km <= 3) dz = dz_free_image(p3, ny, n_free, kdir);
+      if (ry == 1) dy = t_22<JD>(y[c]);
+      if (ry == 0) dy = t_drp<JD>(y[c]);
+      if (rz == 1) dz = t_22<KD>(z[c]);
+      if (rz == 0) dz = t_drp<KD>(z[c]);
+      if (a.isfree == 1 && km <= 3) dz = t_free<KD>(z[c], lo[c], n_free);
       /* image sums (trial_slipweakening.cu:230-256): slot 2,1,0 minus / 4,5,6 plus */
       float rr = (float)(kA1 * t1[c][0] + kA2 * t1[c][1] + kA3 * t1[c][2]);
       R[m][c] = (float)(0.5 * ((2 * m - 1) * rr + (dy + dz)));
@@ -246,23 +322,27 @@ DEVI void k_trial_body(const FaultArgs &a, int id) {
     Trial[c] = (float)(2.0 * (Mrho[0] * Mrho[1] * dV / a.dt + Mrho[0] * R[1][c] - Mrho[1] * R[0][c]) /
                        (kA0 * (Mrho[0] + Mrho[1])));
   }
+  float vs1[3] = {F.vs[pf], F.vs[ss + pf], F.vs[2 * ss + pf]};
+  float vs2[3] = {F.vs[3 * ss + pf], F.vs[4 * ss + pf], F.vs[5 * ss + pf]};
+  float T0[3] = {F.T0[pf], F.T0[ss + pf], F.T0[2 * ss + pf]};
+  float mus = F.fric[pf], mud = F.fric[ss + pf], Dc = F.fric[2 * ss + pf], C0 = F.fric[3 * ss + pf];
+  float Slip = F.out[6 * ss + pf];
+  float o[3] = {0.0f, 0.0f, 0.0f};
+  if (a.istage != 0) { o[0] = F.out[pf]; o[1] = F.out[ss + pf]; o[2] = F.out[2 * ss + pf]; }
   if (a.tape) {
     const int slot = *a.it_dev - a.tape_it0;
     if (slot >= 0 && slot < a.tape_nt) {
       float *tp = a.tape + ((long)id * a.tape_nt + slot) * kTapeFloats * ss + pf;
 #pragma unroll
       for (int c = 0; c < 3; c++) tp[(3 * a.istage + c) * ss] = Trial[c];
-      if (a.istage == 0) tp[12 * ss] = F.out[6 * ss + pf];
+      if (a.istage == 0) tp[12 * ss] = Slip;
     }
   }
-  float vs1[3] = {F.vs[pf], F.vs[ss + pf], F.vs[2 * ss + pf]};
-  float vs2[3] = {F.vs[3 * ss + pf], F.vs[4 * ss + pf], F.vs[5 * ss + pf]};
-  float vn[3] = {F.fmet[ss + pf], F.fmet[2 * ss + pf], F.fmet[3 * ss + pf]};
+  float vn[3] = {fm[1], fm[2], fm[3]};
   float vn0 = norm3(vn);
-  float jacvec = F.fmet[pf] * vn0;
+  float jacvec = fm[0] * vn0;
 #pragma unroll
   for (int c = 0; c < 3; c++) vn[c] /= vn0;
-  float T0[3] = {F.T0[pf], F.T0[ss + pf], F.T0[2 * ss + pf]};
   float TL[3], Ts[3];
 #pragma unroll
   for (int c = 0; c < 3; c++) TL[c] = Trial[c] / jacvec + T0[c];
@@ -274,8 +354,6 @@ DEVI void k_trial_body(const FaultArgs &a, int id) {
   float Tau_n, Tau_s;
   if (Tn0 >= 0.0f) { Tau_n = 0.0f; ifchange = 1; }  /* no opening */
   else Tau_n = Tn0;
-  float mus = F.fric[pf], mud = F.fric[ss + pf], Dc = F.fric[2 * ss + pf], C0 = F.fric[3 * ss + pf];
-  float Slip = F.out[6 * ss + pf];
   float fr = (Slip <= Dc) ? mus - (mus - mud) * Slip / Dc : mud;
   float Tau_c = -fr * Tau_n + C0;
   if (Ts0 >= Tau_c) { Tau_s = Tau_c; F.flag_rup[pf] = 1; ifchange = 1; }
@@ -293,22 +371,26 @@ DEVI void k_trial_body(const FaultArgs &a, int id) {
 #pragma unroll
     for (int c = 0; c < 3; c++) Tau[c] = TL[c];
   }
+  float t1n[3];  /* the fault traction of the stage, T1 slot 3 */
 #pragma unroll
-  for (int c = 0; c < 3; c++)
-    F.T1[(long)c * 7 * ss + 3 * ss + pf] = (ifchange == 1) ? (Tau[c] - T0[c]) * jacvec : Trial[c];
+  for (int c = 0; c < 3; c++) {
+    t1n[c] = (ifchange == 1) ? (Tau[c] - T0[c]) * jacvec : Trial[c];
+    F.T1[(long)c * 7 * ss + 3 * ss + pf] = t1n[c];
+  }
   float tTs1 = dot3(Tau, vs1), tTs2 = dot3(Tau, vs2), tTn = Tau_n;
   if (a.istage == 0) {
     F.out[pf] = a.rkb * tTn; F.out[ss + pf] = a.rkb * tTs1; F.out[2 * ss + pf] = a.rkb * tTs2;
   } else {
-    F.out[pf] += a.rkb * tTn; F.out[ss + pf] += a.rkb * tTs1; F.out[2 * ss + pf] += a.rkb * tTs2;
+    F.out[pf] = o[0] + a.rkb * tTn; F.out[ss + pf] = o[1] + a.rkb * tTs1; F.out[2 * ss + pf] = o[2] + a.rkb * tTs2;
   }
   /* split-node average onto the stage input (transform: fault2wave_onestage(w_cur)) */
-  fault2wave_node(a, F, pf, p0, a.w_cur, fc);
+  fault2wave_node(a, fm, t1n, v, p0, a.w_cur);
 }
 
-__global__ void __launch_bounds__(128) k_trial(FaultArgs a, BatArgs b) {
+template <int JD, int KD>
+__global__ void __launch_bounds__(64) k_trial(FaultArgs a, BatArgs b) {
   const int id = (int)blockIdx.z % a.nfault;
-  k_trial_body(fault_at(a, b, b.act[blockIdx.z / a.nfault]), id);
+  k_trial_body<JD, KD>(fault_at(a, b, b.act[blockIdx.z / a.nfault]), id);
 }
 
 /* Hooke's law on one column point (sv_curv_col_el_iso_fault_gpu.cu:1126-1154) */
@@ -579,7 +661,7 @@ __global__ void __launch_bounds__(64 * kColRows) k_fault_cols(FaultArgs a, BatAr
    the stage output (drv_rk_curv_col.cu:356-359, 541-544) and at the last
    stage the per-step accumulators (fault_var_update_gpu, fault_wav_t.cu:
    197-264). One lane per node, lanes along j. */
-template <int IDIR>
+template <int IDIR, int JD, int KD>
 DEVI void k_fault_nodes_body(const FaultArgs &a, int id) {
   const int iy = blockIdx.x * blockDim.x + threadIdx.x;
   const int iz = blockIdx.y * blockDim.y + threadIdx.y;
@@ -587,39 +669,56 @@ DEVI void k_fault_nodes_body(const FaultArgs &a, int id) {
   const FaultDev F = fdev(a, id);
   const long ss = a.g.sslice, sc = a.g.sicmp, ny = a.g.ny, sy = a.g.siy, sz = a.g.siz;
   const long pf = (iy + 3) + (long)(iz + 3) * ny;
-  if (F.united[pf] != 0) return;
-  const int jdir = a.jdir, kdir = a.kdir;
+  const int united = F.united[pf], ry = F.rupy[pf], rz = F.rupz[pf];
+  if (united != 0) return;
   const int i0 = F.i0;
   const long row = (long)(iy + 3) * sy + (long)(iz + 3) * sz;
   const long p0 = i0 + row;
   const int km = a.g.nk - (iz + 1);
   const int n_free = km + 3;
   const bool surf = (a.isfree == 1);
-  const float *met = a.met;
   const float *W = a.w_cur;
   const float *fc = a.f_cur + (long)id * 18 * ss;
-  const int ry = F.rupy[pf], rz = F.rupz[pf];
   const float *T1 = F.T1;
 
   /* split-node velocity rhs */
-  float fhV[2][3];
+  float fhV[2][3], t1c[3];
+  float jac = F.fmet[pf];
 #pragma unroll
   for (int m = 0; m < 2; m++) {
-    float rrhojac = (float)(1.0 / (F.rho_f[m * ss + pf] * F.fmet[pf]));
+    float rrhojac = (float)(1.0 / (F.rho_f[m * ss + pf] * jac));
+    float y[3][5], z[3][5], tx[3][4];
 #pragma unroll
     for (int c = 0; c < 3; c++) {
       const float *t = T1 + (long)c * 7 * ss + pf;
+      tx[c][0] = t[3 * ss];
+#pragma unroll
+      for (int l = 1; l <= 3; l++) tx[c][l] = t[(3 + (2 * m - 1) * l) * ss];
+      taps5<JD>(fc + fidx(3 + c, m, ss) + pf, 1, y[c]);
+      taps5<KD>(fc + fidx(6 + c, m, ss) + pf, ny, z[c]);
+    }
+    float lo[3][2] = {};
+    if (surf && km == 0 && KD == 1) {
+#pragma unroll
+      for (int c = 0; c < 3; c++) {
+        const float *p3 = fc + fidx(6 + c, m, ss) + pf;
+        lo[c][0] = p3[-3 * ny];
+        lo[c][1] = p3[-2 * ny];
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+      const float *t = tx[c];
+      t1c[c] = t[0];
       float dx;
-      if (m == 0) dx = (float)(kA0 * t[3 * ss] - kA1 * t[2 * ss] - kA2 * t[1 * ss] - kA3 * t[0]);
-      else dx = (float)(-kA0 * t[3 * ss] + kA1 * t[4 * ss] + kA2 * t[5 * ss] + kA3 * t[6 * ss]);
-      const float *p2 = fc + fidx(3 + c, m, ss) + pf;
-      const float *p3 = fc + fidx(6 + c, m, ss) + pf;
+      if (m == 0) dx = (float)(kA0 * t[0] - kA1 * t[1] - kA2 * t[2] - kA3 * t[3]);
+      else dx = (float)(-kA0 * t[0] + kA1 * t[1] + kA2 * t[2] + kA3 * t[3]);
       float dy = 0.0f, dz = 0.0f;
-      if (ry == 1) dy = mac22(p2, 1, jdir);
-      if (ry == 0) dy = macdrp(p2, 1, jdir);
-      if (rz == 1) dz = mac22(p3, ny, kdir);
-      if (rz == 0) dz = macdrp(p3, ny, kdir);
-      if (surf && km <= 3) dz = dz_free_image(p3, ny, n_free, kdir);
+      if (ry == 1) dy = t_22<JD>(y[c]);
+      if (ry == 0) dy = t_drp<JD>(y[c]);
+      if (rz == 1) dz = t_22<KD>(z[c]);
+      if (rz == 0) dz = t_drp<KD>(z[c]);
+      if (surf && km <= 3) dz = t_free<KD>(z[c], lo[c], n_free);
       fhV[m][c] = (dx + dy + dz) * rrhojac;
     }
   }
@@ -629,17 +728,25 @@ DEVI void k_fault_nodes_body(const FaultArgs &a, int id) {
 
   /* split-node velocity gradients: DV[0] minus side, DV[1] plus side */
   const float *V[3] = {W, W + sc, W + 2 * sc};
-  const float *fV[3] = {fc + fidx(0, 0, ss), fc + fidx(1, 0, ss), fc + fidx(2, 0, ss)};
-  const long pm = pf, pp = pf + ss;
-  float DxV[2][3], DyV[2][3], DzV[2][3];
+  float DxV[2][3], DyV[2][3], DzV[2][3], vmid[2][3], Dz2[2][3];
   constexpr int S_ = IDIR == 1 ? 1 : 0;  /* side with the one-sided x difference */
   constexpr int O_ = 1 - S_;
 #pragma unroll
-  for (int c = 0; c < 3; c++) {
-    if (ry == 1) { DyV[1][c] = mac22(fV[c] + pp, 1, jdir); DyV[0][c] = mac22(fV[c] + pm, 1, jdir); }
-    else { DyV[1][c] = macdrp(fV[c] + pp, 1, jdir); DyV[0][c] = macdrp(fV[c] + pm, 1, jdir); }
-    if (rz == 1) { DzV[1][c] = mac22(fV[c] + pp, ny, kdir); DzV[0][c] = mac22(fV[c] + pm, ny, kdir); }
-    else { DzV[1][c] = macdrp(fV[c] + pp, ny, kdir); DzV[0][c] = macdrp(fV[c] + pm, ny, kdir); }
+  for (int m = 1; m >= 0; m--) {
+    float y[3][5], z[3][5];
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+      const float *q = fc + fidx(c, m, ss) + pf;
+      taps5<JD>(q, 1, y[c]);
+      taps5<KD>(q, ny, z[c]);
+    }
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+      vmid[m][c] = t_mid<JD>(y[c]);
+      DyV[m][c] = ry == 1 ? t_22<JD>(y[c]) : t_drp<JD>(y[c]);
+      DzV[m][c] = rz == 1 ? t_22<KD>(z[c]) : t_drp<KD>(z[c]);
+      Dz2[m][c] = km == 1 ? t_22<KD>(z[c]) : t_24<KD>(z[c]);  /* used where km is 1 or 2 */
+    }
   }
   const float *Ms = (IDIR == 1 ? F.P2M : F.M2P) + pf; /* 5 matrices, stride 9*ss between them */
   const float *M2 = F.M2 + pf;                        /* T1toVx,VytoVx,VztoVx (minus), then plus */
@@ -668,8 +775,8 @@ DEVI void k_fault_nodes_body(const FaultArgs &a, int id) {
   if (a.imethod == 1) {
 #pragma unroll
     for (int c = 0; c < 3; c++) {
-      if (IDIR == 1) DxV[1][c] = V[c][(i0 + 1) + row] - fV[c][pp];
-      else DxV[0][c] = fV[c][pm] - V[c][(i0 - 1) + row];
+      if (IDIR == 1) DxV[1][c] = V[c][(i0 + 1) + row] - vmid[1][c];
+      else DxV[0][c] = vmid[0][c] - V[c][(i0 - 1) + row];
     }
     method1();
   } else {
@@ -702,10 +809,7 @@ DEVI void k_fault_nodes_body(const FaultArgs &a, int id) {
   }
   if (surf && (km == 1 || km == 2)) {
 #pragma unroll
-    for (int c = 0; c < 3; c++) {
-      if (km == 1) { DzV[1][c] = mac22(fV[c] + pp, ny, kdir); DzV[0][c] = mac22(fV[c] + pm, ny, kdir); }
-      else { DzV[1][c] = mac24(fV[c] + pp, ny, kdir); DzV[0][c] = mac24(fV[c] + pm, ny, kdir); }
-    }
+    for (int c = 0; c < 3; c++) { DzV[1][c] = Dz2[1][c]; DzV[0][c] = Dz2[0][c]; }
     if (a.imethod == 1) method1();
     else method2();
   }
@@ -731,84 +835,96 @@ DEVI void k_fault_nodes_body(const FaultArgs &a, int id) {
   float *fpre = a.f_pre + (long)id * 18 * ss;
   float *fnew = a.istage < 3 ? a.f_tnew + (long)id * 18 * ss : nullptr;
   float *fend = a.f_end + (long)id * 18 * ss;
-  float fe[2][3];
+  float fm[10];
+  fault_metric_at(F, ss, pf, fm);
+  float pv[9][2], en[9][2];
 #pragma unroll
   for (int m = 0; m < 2; m++)
 #pragma unroll
     for (int c = 0; c < 9; c++) {
-      float r = c < 3 ? fhV[m][c] : (c < 6 ? fhT2[m][c - 3] : fhT3[m][c - 6]);
-      long o = fidx(c, m, ss) + pf;
-      float e;
-      if (a.istage == 0) {
-        float pv = fpre[o];
-        fnew[o] = pv + a.ca * r;
-        e = pv + a.cb * r;
-      } else if (a.istage < 3) {
-        fnew[o] = fpre[o] + a.ca * r;
-        e = fend[o] + a.cb * r;
-      } else {
-        e = fend[o] + a.cb * r;
+      const long o = fidx(c, m, ss) + pf;
+      pv[c][m] = a.istage < 3 ? fpre[o] : 0.0f;
+      en[c][m] = a.istage > 0 ? fend[o] : 0.0f;
+    }
+#pragma unroll
+  for (int m = 0; m < 2; m++)
+#pragma unroll
+    for (int c = 0; c < 9; c++) {
+      const float r = c < 3 ? fhV[m][c] : (c < 6 ? fhT2[m][c - 3] : fhT3[m][c - 6]);
+      const long o = fidx(c, m, ss) + pf;
+      const float e = (a.istage == 0 ? pv[c][m] : en[c][m]) + a.cb * r;
+      if (a.istage < 3) {
+        pv[c][m] = pv[c][m] + a.ca * r;
+        fnew[o] = pv[c][m];
       }
       fend[o] = e;
-      if (c < 3) fe[m][c] = e;
+      en[c][m] = e;
     }
-  if (a.istage < 3) fault2wave_node(a, F, pf, p0, a.w_tnew, fnew);
-  else fault2wave_node(a, F, pf, p0, a.w_end, fend);
+  if (a.istage < 3) {
+    fault2wave_node(a, fm, t1c, pv, p0, a.w_tnew);
+    return;
+  }
+  fault2wave_node(a, fm, t1c, en, p0, a.w_end);
 
-  if (a.istage == 3) {
-    /* per-step accumulators (fault_var_update_gpu, fault_wav_t.cu:219-262) */
-    float dV[3];
+  /* the last stage: per-step accumulators (fault_var_update_gpu, fault_wav_t.cu:219-262) */
+  float vs[6], mT[3];
 #pragma unroll
-    for (int c = 0; c < 3; c++) dV[c] = fe[1][c] - fe[0][c];
-    if (a.tape) {
-      const int slot = *a.it_dev - a.tape_it0;
-      if (slot >= 0 && slot < a.tape_nt) {
-        float *tp = a.tape + ((long)id * a.tape_nt + slot) * kTapeFloats * ss + pf;
+  for (int c = 0; c < 6; c++) vs[c] = F.vs[c * ss + pf];
+  double *sd = F.slip64;
+  const double d0 = sd[pf], d1 = sd[ss + pf], d2 = sd[2 * ss + pf];
 #pragma unroll
-        for (int c = 0; c < 3; c++) tp[(13 + c) * ss] = dV[c];
-      }
-    }
-    float Vs1 = dV[0] * F.vs[pf] + dV[1] * F.vs[ss + pf] + dV[2] * F.vs[2 * ss + pf];
-    float Vs2 = dV[0] * F.vs[3 * ss + pf] + dV[1] * F.vs[4 * ss + pf] + dV[2] * F.vs[5 * ss + pf];
-    float Vs = sqrtf(Vs2 * Vs2 + Vs1 * Vs1);
-    float dt = a.dt;
-    F.out[3 * ss + pf] = Vs;
-    F.out[4 * ss + pf] = Vs1;
-    F.out[5 * ss + pf] = Vs2;
-    /* Slip, Slip1, Slip2 accumulate in FP64; the outputs (and the Slip the
-       friction law reads) are their FP32 values */
-    {
-      double *sd = F.slip64;
-      const double s0 = sd[pf] + (double)(Vs * dt), s1 = sd[ss + pf] + (double)(Vs1 * dt),
-                   s2 = sd[2 * ss + pf] + (double)(Vs2 * dt);
-      sd[pf] = s0;
-      sd[ss + pf] = s1;
-      sd[2 * ss + pf] = s2;
-      F.out[6 * ss + pf] = (float)s0;
-      F.out[7 * ss + pf] = (float)s1;
-      F.out[8 * ss + pf] = (float)s2;
-    }
+  for (int c = 0; c < 3; c++) mT[c] = F.mT1[c * ss + pf];
+  const float peak = F.out[9 * ss + pf];
+  const int t0set = F.init_t0_flag[pf];
+  const int it = *a.it_dev;
+  float dV[3];
 #pragma unroll
-    for (int c = 0; c < 3; c++) {
-      float t = T1[(long)c * 7 * ss + 3 * ss + pf];
-      F.hT1[c * ss + pf] = (t - F.mT1[c * ss + pf]) / dt;
-      F.mT1[c * ss + pf] = t;
+  for (int c = 0; c < 3; c++) dV[c] = en[c][1] - en[c][0];
+  if (a.tape) {
+    const int slot = it - a.tape_it0;
+    if (slot >= 0 && slot < a.tape_nt) {
+      float *tp = a.tape + ((long)id * a.tape_nt + slot) * kTapeFloats * ss + pf;
+#pragma unroll
+      for (int c = 0; c < 3; c++) tp[(13 + c) * ss] = dV[c];
     }
-    if (Vs > F.out[9 * ss + pf]) F.out[9 * ss + pf] = Vs;
-    if (F.init_t0_flag[pf] == 0) {
-      if (Vs > 1e-3) {
-        F.out[10 * ss + pf] = (float)((*a.it_dev + 1) * (double)dt);
-        F.init_t0_flag[pf] = 1;
-        F.flag_rup[pf] = 1;
-      }
+  }
+  float Vs1 = dV[0] * vs[0] + dV[1] * vs[1] + dV[2] * vs[2];
+  float Vs2 = dV[0] * vs[3] + dV[1] * vs[4] + dV[2] * vs[5];
+  float Vs = sqrtf(Vs2 * Vs2 + Vs1 * Vs1);
+  float dt = a.dt;
+  F.out[3 * ss + pf] = Vs;
+  F.out[4 * ss + pf] = Vs1;
+  F.out[5 * ss + pf] = Vs2;
+  /* Slip, Slip1, Slip2 accumulate in FP64; the outputs (and the Slip the
+     friction law reads) are their FP32 values */
+  {
+    const double s0 = d0 + (double)(Vs * dt), s1 = d1 + (double)(Vs1 * dt), s2 = d2 + (double)(Vs2 * dt);
+    sd[pf] = s0;
+    sd[ss + pf] = s1;
+    sd[2 * ss + pf] = s2;
+    F.out[6 * ss + pf] = (float)s0;
+    F.out[7 * ss + pf] = (float)s1;
+    F.out[8 * ss + pf] = (float)s2;
+  }
+#pragma unroll
+  for (int c = 0; c < 3; c++) {
+    F.hT1[c * ss + pf] = (t1c[c] - mT[c]) / dt;
+    F.mT1[c * ss + pf] = t1c[c];
+  }
+  if (Vs > peak) F.out[9 * ss + pf] = Vs;
+  if (t0set == 0) {
+    if (Vs > 1e-3) {
+      F.out[10 * ss + pf] = (float)((it + 1) * (double)dt);
+      F.init_t0_flag[pf] = 1;
+      F.flag_rup[pf] = 1;
     }
   }
 }
 
-template <int IDIR>
-__global__ void __launch_bounds__(256) k_fault_nodes(FaultArgs a, BatArgs b) {
+template <int IDIR, int JD, int KD>
+__global__ void __launch_bounds__(64) k_fault_nodes(FaultArgs a, BatArgs b) {
   const int id = (int)blockIdx.z % a.nfault;
-  k_fault_nodes_body<IDIR>(fault_at(a, b, b.act[blockIdx.z / a.nfault]), id);
+  k_fault_nodes_body<IDIR, JD, KD>(fault_at(a, b, b.act[blockIdx.z / a.nfault]), id);
 }
 
 /* ---------------------------------------------------------------------- */
@@ -874,20 +990,33 @@ void launch_trial(const FaultArgs &a, const BatArgs &b, hipStream_t st) {
   if (a.nfault <= 0) return;
   dim3 tblk(64, 4, 1), tgrd((a.g.nj + kTrialNodes - 1) / kTrialNodes, (a.g.nk + 3) / 4, a.nfault * b.nact);
   hipLaunchKernelGGL(k_trial_t1, tgrd, tblk, 0, st, a, b);
-  dim3 blk(64, 2, 1), grd((a.g.nj + 63) / 64, (a.g.nk + 1) / 2, a.nfault * b.nact);
-  hipLaunchKernelGGL(k_trial, grd, blk, 0, st, a, b);
+  dim3 blk(64, 1, 1), grd((a.g.nj + 63) / 64, a.g.nk, a.nfault * b.nact);
+  switch (a.jdir * 2 + a.kdir) {
+    case 0: hipLaunchKernelGGL((k_trial<0, 0>), grd, blk, 0, st, a, b); break;
+    case 1: hipLaunchKernelGGL((k_trial<0, 1>), grd, blk, 0, st, a, b); break;
+    case 2: hipLaunchKernelGGL((k_trial<1, 0>), grd, blk, 0, st, a, b); break;
+    default: hipLaunchKernelGGL((k_trial<1, 1>), grd, blk, 0, st, a, b); break;
+  }
 }
 void launch_fault_update(const FaultArgs &a, const BatArgs &b, hipStream_t st) {
   if (a.nfault <= 0) return;
   dim3 cblk(64, kColRows, 1),
       cgrd((a.g.nj + kColNodes - 1) / kColNodes, (a.g.nk + kColRows - 1) / kColRows, a.nfault * b.nact);
-  dim3 nblk(64, 4, 1), ngrd((a.g.nj + 63) / 64, (a.g.nk + 3) / 4, a.nfault * b.nact);
+  dim3 nblk(64, 1, 1), ngrd((a.g.nj + 63) / 64, a.g.nk, a.nfault * b.nact);
   if (a.idir == 1) {
     hipLaunchKernelGGL(k_fault_cols<1>, cgrd, cblk, 0, st, a, b);
-    hipLaunchKernelGGL(k_fault_nodes<1>, ngrd, nblk, 0, st, a, b);
   } else {
     hipLaunchKernelGGL(k_fault_cols<0>, cgrd, cblk, 0, st, a, b);
-    hipLaunchKernelGGL(k_fault_nodes<0>, ngrd, nblk, 0, st, a, b);
+  }
+  switch (a.idir * 4 + a.jdir * 2 + a.kdir) {
+    case 0: hipLaunchKernelGGL((k_fault_nodes<0, 0, 0>), ngrd, nblk, 0, st, a, b); break;
+    case 1: hipLaunchKernelGGL((k_fault_nodes<0, 0, 1>), ngrd, nblk, 0, st, a, b); break;
+    case 2: hipLaunchKernelGGL((k_fault_nodes<0, 1, 0>), ngrd, nblk, 0, st, a, b); break;
+    case 3: hipLaunchKernelGGL((k_fault_nodes<0, 1, 1>), ngrd, nblk, 0, st, a, b); break;
+    case 4: hipLaunchKernelGGL((k_fault_nodes<1, 0, 0>), ngrd, nblk, 0, st, a, b); break;
+    case 5: hipLaunchKernelGGL((k_fault_nodes<1, 0, 1>), ngrd, nblk, 0, st, a, b); break;
+    case 6: hipLaunchKernelGGL((k_fault_nodes<1, 1, 0>), ngrd, nblk, 0, st, a, b); break;
+    default: hipLaunchKernelGGL((k_fault_nodes<1, 1, 1>), ngrd, nblk, 0, st, a, b); break;
   }
 }
 void launch_step_end(int *it_dev, hipStream_t st) { hipLaunchKernelGGL(k_step_end, dim3(1), dim3(64), 0, st, it_dev); }
