@@ -540,6 +540,16 @@ __global__ void __launch_bounds__(256, 5) k_vol_bat_pml_band(VolArgs a, BatArgs 
   pml_acc_point<ID, JD, KD, VC, DM>(a, b, i, j, k, b.act[sq]);
 }
 
+/* Largest plane of the interior box (points) for the one-launch form, which
+   runs the box plane by plane and at the bands' 5 waves per SIMD instead of
+   8. A batch takes it on vertical columns alone; with nine metric terms its
+   bands stay in the groups of variant 32, whose sums round differently.
+   Against the two kernels: 0.674 against 0.693 ms per stage at 200 x 400 x
+   150 (a plane of 45800 points); at 260 x 400 x 80 (68700, nine metric terms)
+   3% slower, at 400 x 800 x 266 (243000: the planes under way outgrow the L2s
+   without slab order) 4.61 against 4.09 ms. */
+constexpr long kOneLaunchPlane = 48000;
+
 constexpr int kBandSlabBlocks = 192;
 
 /* the bands in groups by the CFS-PML face directions their points can lie
@@ -612,6 +622,36 @@ static void box_split(const VolArgs &a, int tw, bool grouped, VolBox &x, VolBand
   add(2, xl, xr, yr, g.nj + 3, kr, kv1);
   add(3, xl, xr, yl, yr, kv0, kl);
   add(3, xl, xr, yl, yr, kr, kv1);
+}
+
+/* The box split in one launch (variants 32 and 33 where a plane of the
+   interior box is small): block ids [0, nband) of a scenario's per are the
+   bands (the longer blocks first), the rest the box in TW x 256/TW tiles, x
+   tile fastest, then y, then the plane. On such grids either kernel alone is
+   one or two rounds of resident blocks, and one launch fills the bands' last
+   round with box tiles: 55.5 -> 47.6 us per stage at 80 x 120 x 60, 91.6 ->
+   82.2 at 96 x 141 x 72, 253 -> 243 at 160 x 240 x 100, 693 -> 674 at 200 x
+   400 x 150, six scenarios at 80 x 120 x 60 296 -> 244, twelve at 200 x 400 x
+   150 8.12 -> 7.91 ms. 32-wide tiles unless the box is whole 64-column tiles
+   (its x bounds are multiples of 32; 48.4 against 47.1 us at 80 x 120 x 60). */
+template <int ID, int JD, int KD, int TW, bool VC>
+__global__ void __launch_bounds__(256, 5) k_vol_split(VolArgs a, BatArgs b, VolBox x, VolBands r, unsigned per) {
+  const int sn = b.act[blockIdx.x / per];
+  const unsigned nband = (unsigned)r.cum[r.n];
+  unsigned L = blockIdx.x % per;
+  int i, j, k;
+  if (L < nband) {
+    if (!band_point(r, L, i, j, k)) return;
+    pml_acc_point<ID, JD, KD, VC, 7>(a, b, i, j, k, sn);
+    return;
+  }
+  L -= nband;
+  const int t = (int)threadIdx.x;
+  i = x.x0 + (int)(L % (unsigned)x.ntx) * TW + (t % TW);
+  L /= (unsigned)x.ntx;
+  j = x.y0 + (int)(L % (unsigned)x.nty) * (256 / TW) + t / TW;
+  if (i >= x.x1 || j >= x.y1) return;
+  acc_point<ID, JD, KD, 1, VC>(a, b, i, j, x.k0 + (int)(L / (unsigned)x.nty), sn);
 }
 
 template <int ID, int JD, int KD, bool VC, int G>
@@ -925,10 +965,28 @@ __global__ void k_pg(Grid g, BatArgs b, const float *__restrict__ wend, const fl
 /* the box split (variants 23, 64-wide interior tiles, 24, 32-wide, and 33,
    23 with every band in one launch): one scenario or a batch */
 template <int ID, int JD, int KD, bool VC>
-static void launch_box_split(int tw, bool sweeps, bool grouped, const VolArgs &a, const BatArgs &b, hipStream_t st,
+static void launch_box_split(int tw, bool sweeps, bool grouped, bool one, const VolArgs &a, const BatArgs &b, hipStream_t st,
                              hipStream_t st_pml) {
   VolBox x;
   VolBands r[kBandGroups];
+  if (one) {
+    box_split(a, 64, false, x, r);
+    const int w = x.x1 - x.x0;
+    const bool plane = (long)w * (x.y1 - x.y0) <= kOneLaunchPlane && st == st_pml && (VC || !grouped);
+    /* 32-wide tiles where 64-wide ones would idle more than a tenth of their
+       lanes (a box of 224 columns, 300 x 500 x 80: 3% off the step) */
+    if (10 * w < 9 * 64 * x.ntx && (plane || b.nact == 1)) tw = 32;
+    if (plane) {
+      if (tw == 32) box_split(a, 32, false, x, r);
+      const unsigned per = (unsigned)((long)x.ntx * x.nty * (x.k1 - x.k0) + r[0].cum[r[0].n]);
+      const dim3 grd(per * (unsigned)b.nact);
+      if (tw == 64)
+        hipLaunchKernelGGL((k_vol_split<ID, JD, KD, 64, VC>), grd, dim3(256), 0, st, a, b, x, r[0], per);
+      else
+        hipLaunchKernelGGL((k_vol_split<ID, JD, KD, 32, VC>), grd, dim3(256), 0, st, a, b, x, r[0], per);
+      return;
+    }
+  }
   box_split(a, tw, grouped, x, r);
   if (b.nact > 1 && sweeps && x.ntx > 0) {  /* variant 32: per-scenario slab sweeps of the box (64 x 4 tiles) */
     const long nslab = ((long)x.nty + a.zchunk - 1) / a.zchunk;
@@ -970,8 +1028,9 @@ static void launch_dir(int variant, const VolArgs &a, const BatArgs &b, int top,
   if (variant == 23 || variant == 24 || variant == 32 || variant == 33) {
     const int tw = variant == 24 ? 32 : 64;
     const bool grouped = variant != 33;
-    if (a.vcol) launch_box_split<ID, JD, KD, true>(tw, variant == 32, grouped, a, b, st, st_pml);
-    else launch_box_split<ID, JD, KD, false>(tw, variant == 32, grouped, a, b, st, st_pml);
+    const bool one = variant == 32 || variant == 33;
+    if (a.vcol) launch_box_split<ID, JD, KD, true>(tw, variant == 32, grouped, one, a, b, st, st_pml);
+    else launch_box_split<ID, JD, KD, false>(tw, variant == 32, grouped, one, a, b, st, st_pml);
     return;
   }
   if (b.nact > 1 && variant == 20) {  /* batches, split kernels */

@@ -339,7 +339,11 @@ int cgfd_core_run_timed(cgfd_core *core, int nsteps, float *ms_total,
    order) and the lean PML kernel over the up to six slabs around them in
    32 x 8 tiles, launched in up to four groups by the CFS-PML face
    directions their points can lie in; 32 = 23 on one scenario; 33 = 23
-   with every band in one launch that handles all three directions. Batches with more than one active
+   with every band in one launch that handles all three directions, and,
+   where a plane of the box has at most 48000 points, the box in that launch
+   too (a batch on 32 or 33 as well, on vertical columns; not under the stage
+   fork); 33 takes 32-wide tiles where 64-wide ones would idle over a tenth
+   of their lanes. Batches with more than one active
    scenario run, for 20, the interior tiles with the scenarios back to back
    (XCD-contiguous) and the PML tiles in one slab-ordered sweep per
    scenario; for 23, 24 and 33 the box split the same way (interior tiles with
@@ -353,7 +357,8 @@ int cgfd_core_set_variant(cgfd_core *core, int variant);
    been resolved). */
 int cgfd_core_get_variant(const cgfd_core *core, int *variant, int *zchunk);
 
-/* y-tiles per slab of the slab-ordered kernels (20, 23, 24, 32, 33), 4..4096. */
+/* y-tiles per slab of the slab-ordered kernels (20, 23, 24, 32, 33), 4..4096;
+   without effect where 32 and 33 run as one launch. */
 int cgfd_core_set_zchunk(cgfd_core *core, int zchunk);
 
 /* Vertical-column metric form, no counterpart in the reference (whose
