@@ -78,6 +78,14 @@ DEVI long face_idx(const AdjFace &F, int i, int j, int k) {
   return (long)(k - F.k1) * ((long)F.bn * F.an) + (long)(j - F.j1) * F.an + (i - F.ax0);
 }
 
+/* Tiles of the three kernels start at ghost-inclusive column 0, as the
+   forward kernels' do: a 64-lane row of any array is then two whole 128-byte
+   lines instead of parts of three, and one more tile for the last columns
+   when ni mod 64 is 0, 62 or 63 moves no more lines than the row did before.
+   160x240x100: k_adj_prep 200 -> 175 us, k_adj_stage 325 -> 258 us. */
+constexpr int kTileW = 64;
+static unsigned tiles_x(const Grid &g) { return (unsigned)((g.ni + 3 + kTileW - 1) / kTileW); }
+
 /* S and G from c = alpha X + beta E at physical points (X may be null);
    at CFS-PML points also the per-face extra S and G and the auxiliaries'
    reverse stage (MODE as k_adj_stage) */
@@ -86,9 +94,9 @@ __global__ void __launch_bounds__(256) k_adj_prep(Grid g, const float *__restric
                                                   const float *__restrict__ slw, const float *__restrict__ X,
                                                   float alpha, const float *__restrict__ E, float beta,
                                                   float *__restrict__ SG, AdjPml pm, int isfree, int kdir) {
-  const int i = blockIdx.x * 64 + (int)threadIdx.x + 3, j = blockIdx.y * 4 + (int)threadIdx.y + 3;
+  const int i = blockIdx.x * kTileW + (int)threadIdx.x, j = blockIdx.y * 4 + (int)threadIdx.y + 3;
   const int k = (int)blockIdx.z + 3;
-  if (i >= g.ni + 3 || j >= g.nj + 3) return;
+  if (i < 3 || i >= g.ni + 3 || j >= g.nj + 3) return;
   const long sc = g.sicmp;
   const long p = i + j * g.siy + (long)k * g.siz;
   if (pm.fs.nfault > 0 && fault_column(pm.fs, i, j + (long)k * g.ny)) {
@@ -123,17 +131,27 @@ __global__ void __launch_bounds__(256) k_adj_prep(Grid g, const float *__restric
     float *Pa = F.lev + (long)pm.lp * 9 * n;
     float *Aw = F.lev + 9 * n, *Bw = F.lev + 18 * n;
     const float *Xa = MODE == 3 ? nullptr : (MODE == 1 ? Ba : Aa);
-    float dc[9];
+    /* loads before stores, which may alias them for all the compiler knows: one
+       wait per face instead of one per component */
+    float dc[9], ev[9], xv[9], av[9], pv[9];
 #pragma unroll
     for (int f = 0; f < 9; f++) {
       const long o2 = f * n + ia;
-      const float ca_ = beta * Ea[o2] + (Xa ? alpha * Xa[o2] : 0.0f);  /* auxiliary rhs adjoint */
+      ev[f] = Ea[o2];
+      xv[f] = Xa ? Xa[o2] : 0.0f;
+      av[f] = MODE == 2 || MODE == 0 ? Aa[o2] : (MODE == 1 ? Ba[o2] : 0.0f);
+      pv[f] = MODE < 2 ? Pa[o2] : 0.0f;
+    }
+#pragma unroll
+    for (int f = 0; f < 9; f++) {
+      const long o2 = f * n + ia;
+      const float ca_ = beta * ev[f] + (Xa ? alpha * xv[f] : 0.0f);  /* auxiliary rhs adjoint */
       dc[f] = (cB - 1.0f) * c[f] + cD * ca_;
       const float la = -cB * c[f] - cA * ca_;                          /* auxiliary stage adjoint */
       if (MODE == 3) Aw[o2] = la;
-      else if (MODE == 2) { Bw[o2] = la; Pa[o2] = Ea[o2] + Aa[o2]; }
-      else if (MODE == 1) { const float b = Ba[o2]; Aw[o2] = la; Pa[o2] += b; }
-      else Pa[o2] += Aa[o2] + la;
+      else if (MODE == 2) { Bw[o2] = la; Pa[o2] = ev[f] + av[f]; }
+      else if (MODE == 1) { Aw[o2] = la; Pa[o2] = pv[f] + av[f]; }
+      else Pa[o2] = pv[f] + (av[f] + la);
     }
     sg_of(dc, l, m, s, o);
 #pragma unroll
@@ -147,102 +165,134 @@ DEVI float tap_coef(int t) {
              : (t == 0 ? CGFD_CB0 : t == 1 ? CGFD_CB1 : t == 2 ? CGFD_CB2 : t == 3 ? CGFD_CB3 : CGFD_CB4);
 }
 
-/* add w * kappa(., d)(p) for all nine fields; M: metric row d at p.
-   AX = 0 or 1: only M[AX] is nonzero (the xi and eta rows on a grid of
-   vertical columns, see acc_core), and only the S and G entries it
-   multiplies are read; AX = -1: the full row */
+/* S and G (and nothing else) of one tap; the entries the direction's metric
+   row multiplies. AX = 0 or 1: only M[AX] is nonzero (the xi and eta rows on a
+   grid of vertical columns, see acc_core); AX = -1: the full row */
 template <int AX>
-DEVI void add_kappa(float *lm, float w, const float *__restrict__ SG, long sc, long p, float M0, float M1, float M2) {
-  const float Sx = SG[p], Sy = SG[sc + p], Sz = SG[2 * sc + p];
-  const float *G = SG + 3 * sc + p;  /* xx, yy, zz, xy, xz, yz (sg_of) */
+DEVI void load_sg(float *g, const float *__restrict__ SG, long sc, long p) {
+#pragma unroll
+  for (int q = 0; q < kSG; q++)
+    if (AX == -1 || q < 3 || (AX == 0 && (q == 3 || q == 6 || q == 7)) || (AX == 1 && (q == 4 || q == 6 || q == 8)))
+      g[q] = SG[q * sc + p];
+}
+/* add w * kappa(., d) for all nine fields from a tap's S and G (g) and metric
+   row (M) */
+template <int AX>
+DEVI void add_kappa(float *lm, float w, const float *g, const float *M) {
   if (AX == 0) {
-    lm[VX] += w * (M0 * G[0]);
-    lm[VY] += w * (M0 * G[3 * sc]);
-    lm[VZ] += w * (M0 * G[4 * sc]);
-    lm[TXX] += w * (M0 * Sx);
-    lm[TXY] += w * (M0 * Sy);
-    lm[TXZ] += w * (M0 * Sz);
+    const float u = w * M[0];
+    lm[VX] += u * g[3];
+    lm[VY] += u * g[6];
+    lm[VZ] += u * g[7];
+    lm[TXX] += u * g[0];
+    lm[TXY] += u * g[1];
+    lm[TXZ] += u * g[2];
   } else if (AX == 1) {
-    lm[VX] += w * (M1 * G[3 * sc]);
-    lm[VY] += w * (M1 * G[sc]);
-    lm[VZ] += w * (M1 * G[5 * sc]);
-    lm[TYY] += w * (M1 * Sy);
-    lm[TXY] += w * (M1 * Sx);
-    lm[TYZ] += w * (M1 * Sz);
+    const float u = w * M[1];
+    lm[VX] += u * g[6];
+    lm[VY] += u * g[4];
+    lm[VZ] += u * g[8];
+    lm[TYY] += u * g[1];
+    lm[TXY] += u * g[0];
+    lm[TYZ] += u * g[2];
   } else {
-    const float Gxx = G[0], Gyy = G[sc], Gzz = G[2 * sc], Gxy = G[3 * sc], Gxz = G[4 * sc], Gyz = G[5 * sc];
-    lm[VX] += w * (M0 * Gxx + M1 * Gxy + M2 * Gxz);
-    lm[VY] += w * (M0 * Gxy + M1 * Gyy + M2 * Gyz);
-    lm[VZ] += w * (M0 * Gxz + M1 * Gyz + M2 * Gzz);
-    lm[TXX] += w * (M0 * Sx);
-    lm[TYY] += w * (M1 * Sy);
-    lm[TZZ] += w * (M2 * Sz);
-    lm[TXY] += w * (M0 * Sy + M1 * Sx);
-    lm[TXZ] += w * (M0 * Sz + M2 * Sx);
-    lm[TYZ] += w * (M1 * Sz + M2 * Sy);
+    lm[VX] += w * (M[0] * g[3] + M[1] * g[6] + M[2] * g[7]);
+    lm[VY] += w * (M[0] * g[6] + M[1] * g[4] + M[2] * g[8]);
+    lm[VZ] += w * (M[0] * g[7] + M[1] * g[8] + M[2] * g[5]);
+    lm[TXX] += w * (M[0] * g[0]);
+    lm[TYY] += w * (M[1] * g[1]);
+    lm[TZZ] += w * (M[2] * g[2]);
+    lm[TXY] += w * (M[0] * g[1] + M[1] * g[0]);
+    lm[TXZ] += w * (M[0] * g[2] + M[2] * g[0]);
+    lm[TYZ] += w * (M[1] * g[2] + M[2] * g[1]);
   }
 }
 
-/* the per-face extra S and G of the faces along `dim` at tap (ti, tj, tk) */
-template <int AX>
-DEVI void add_face_kappa(float *lm, float w, const AdjPml &pm, int dim, int ti, int tj, int tk, float M0, float M1,
-                         float M2) {
+/* the transposed operator along D (operator direction FW): the five taps'
+   metric rows and S, G are loaded together, and only then, where a tap lies
+   in a CFS-PML face of this direction, the faces' extra S and G, again
+   together. (With the faces tested tap by tap the kernel waited for memory
+   at every tap.) */
+template <int D, int FW, int AX>
+DEVI void gather_dir(float *lm, const Grid &g, const float *__restrict__ met, const float *__restrict__ SG,
+                     const AdjPml &pm, int i, int j, int k, long q) {
+  constexpr int o0 = FW ? -1 : -3;
+  const long sc = g.sicmp, st = D == 0 ? 1 : (D == 1 ? g.siy : g.siz);
+  float M[5][3], s[5][kSG];
 #pragma unroll
+  for (int t = 0; t < 5; t++) {
+    const long p = q - (o0 + t) * st;
+#pragma unroll
+    for (int c = 0; c < 3; c++) M[t][c] = AX == -1 || AX == c ? met[(1 + 3 * D + c) * sc + p] : 0.0f;
+    load_sg<AX>(s[t], SG, sc, p);
+  }
+#pragma unroll
+  for (int t = 0; t < 5; t++) add_kappa<AX>(lm, tap_coef<FW>(t), s[t], M[t]);
+  if (!pm.on) return;
+  const int x = D == 0 ? i : (D == 1 ? j : k);
+#pragma unroll 1
   for (int side = 0; side < 2; side++) {
-    const AdjFace &F = pm.f[2 * dim + side];
-    if (!in_face(F, ti, tj, tk)) continue;
-    add_kappa<AX>(lm, w, F.dsg, F.n, face_idx(F, ti, tj, tk), M0, M1, M2);
+    const AdjFace &F = pm.f[2 * D + side];
+    if (!F.on) continue;
+    const int lo = D == 0 ? F.i1 : (D == 1 ? F.j1 : F.k1), hi = D == 0 ? F.i2 : (D == 1 ? F.j2 : F.k2);
+    /* some tap x - o0 - t, t = 0..4, in [lo, hi], and the other coordinates in the face */
+    const bool near = x - o0 >= lo && x - o0 - 4 <= hi && (D == 0 || (i >= F.i1 && i <= F.i2)) &&
+                      (D == 1 || (j >= F.j1 && j <= F.j2)) && (D == 2 || (k >= F.k1 && k <= F.k2));
+    if (!near) continue;
+    const long fs = D == 0 ? 1 : (D == 1 ? (long)F.an : (long)F.bn * F.an), f0 = face_idx(F, i, j, k);
+#pragma unroll
+    for (int t = 0; t < 5; t++) {
+      const int tx = x - (o0 + t);
+      const bool in = tx >= lo && tx <= hi;
+#pragma unroll
+      for (int e = 0; e < kSG; e++) s[t][e] = 0.0f;
+      if (in) load_sg<AX>(s[t], F.dsg, F.n, f0 - (o0 + t) * fs);
+    }
+#pragma unroll
+    for (int t = 0; t < 5; t++) add_kappa<AX>(lm, tap_coef<FW>(t), s[t], M[t]);
   }
 }
 
 /* MODE 3: A = L^T;  2: B = L^T, P = E + A;  1: A = L^T, P += B;  0: P += A + L^T.
    VC: vertical columns (xi_y, xi_z, eta_x, eta_z left out, as the forward
-   box split does) */
+   box split does).
+   Bound by the L1 misses a CU can have in flight, so the 2 x 2 rows of a
+   block share taps both ways: 160x240x100 258 us as 4 x 1 rows, 250 as 2 x 2;
+   50x71x40 16.0, 14.5; 80x128x48 30.6, 31.7. */
 template <int ID, int JD, int KD, int MODE, bool VC>
-__global__ void __launch_bounds__(256) k_adj_stage(Grid g, const float *__restrict__ met,
+__global__ void __launch_bounds__(256, 4) k_adj_stage(Grid g, const float *__restrict__ met,
                                                    const float *__restrict__ SG, const float *__restrict__ E,
                                                    float *A, float *B, float *P, AdjPml pm) {
-  const int i = blockIdx.x * 64 + (int)threadIdx.x + 3, j = blockIdx.y * 4 + (int)threadIdx.y + 3;
-  const int k = (int)blockIdx.z + 3;
-  if (i >= g.ni + 3 || j >= g.nj + 3) return;
+  const int i = blockIdx.x * kTileW + (int)threadIdx.x, j = blockIdx.y * 2 + (int)threadIdx.y + 3;
+  const int k = (int)(blockIdx.z * 2 + threadIdx.z) + 3;
+  if (i < 3 || i >= g.ni + 3 || j >= g.nj + 3 || k > g.nk2) return;
   const long sc = g.sicmp, sy = g.siy, sz = g.siz;
   const long q = i + j * sy + (long)k * sz;
   float lm[9];
 #pragma unroll
   for (int f = 0; f < 9; f++) lm[f] = 0.0f;
-  constexpr int ox = ID ? -1 : -3, oy = JD ? -1 : -3, oz = KD ? -1 : -3;
-#pragma unroll
-  for (int t = 0; t < 5; t++) {
-    const long p = q - (ox + t);
-    const float M0 = met[sc + p], M1 = VC ? 0.0f : met[2 * sc + p], M2 = VC ? 0.0f : met[3 * sc + p];
-    add_kappa<VC ? 0 : -1>(lm, tap_coef<ID>(t), SG, sc, p, M0, M1, M2);
-    if (pm.on) add_face_kappa<VC ? 0 : -1>(lm, tap_coef<ID>(t), pm, 0, i - (ox + t), j, k, M0, M1, M2);
-  }
+  gather_dir<0, ID, VC ? 0 : -1>(lm, g, met, SG, pm, i, j, k, q);
   __asm__ volatile("" : "+v"(lm[0]), "+v"(lm[1]), "+v"(lm[2]), "+v"(lm[3]), "+v"(lm[4]), "+v"(lm[5]),
                    "+v"(lm[6]), "+v"(lm[7]), "+v"(lm[8]) : : "memory");
-#pragma unroll
-  for (int t = 0; t < 5; t++) {
-    const long p = q - (long)(oy + t) * sy;
-    const float M0 = VC ? 0.0f : met[4 * sc + p], M1 = met[5 * sc + p], M2 = VC ? 0.0f : met[6 * sc + p];
-    add_kappa<VC ? 1 : -1>(lm, tap_coef<JD>(t), SG, sc, p, M0, M1, M2);
-    if (pm.on) add_face_kappa<VC ? 1 : -1>(lm, tap_coef<JD>(t), pm, 1, i, j - (oy + t), k, M0, M1, M2);
-  }
+  gather_dir<1, JD, VC ? 1 : -1>(lm, g, met, SG, pm, i, j, k, q);
   __asm__ volatile("" : "+v"(lm[0]), "+v"(lm[1]), "+v"(lm[2]), "+v"(lm[3]), "+v"(lm[4]), "+v"(lm[5]),
                    "+v"(lm[6]), "+v"(lm[7]), "+v"(lm[8]) : : "memory");
+  gather_dir<2, KD, -1>(lm, g, met, SG, pm, i, j, k, q);
+  /* loads before stores */
+  float av[9], pv[9];
 #pragma unroll
-  for (int t = 0; t < 5; t++) {
-    const long p = q - (long)(oz + t) * sz;
-    const float M0 = met[7 * sc + p], M1 = met[8 * sc + p], M2 = met[9 * sc + p];
-    add_kappa<-1>(lm, tap_coef<KD>(t), SG, sc, p, M0, M1, M2);
-    if (pm.on) add_face_kappa<-1>(lm, tap_coef<KD>(t), pm, 2, i, j, k - (oz + t), M0, M1, M2);
+  for (int f = 0; f < 9; f++) {
+    const long o = f * sc + q;
+    av[f] = MODE == 2 || MODE == 0 ? A[o] : (MODE == 1 ? B[o] : 0.0f);
+    pv[f] = MODE == 2 ? E[o] : (MODE < 2 ? P[o] : 0.0f);
   }
 #pragma unroll
   for (int f = 0; f < 9; f++) {
     const long o = f * sc + q;
     if (MODE == 3) A[o] = lm[f];
-    else if (MODE == 2) { B[o] = lm[f]; P[o] = E[o] + A[o]; }
-    else if (MODE == 1) { const float b = B[o]; A[o] = lm[f]; P[o] += b; }
-    else P[o] += A[o] + lm[f];
+    else if (MODE == 2) { B[o] = lm[f]; P[o] = pv[f] + av[f]; }
+    else if (MODE == 1) { A[o] = lm[f]; P[o] = pv[f] + av[f]; }
+    else P[o] = pv[f] + (av[f] + lm[f]);
   }
 }
 
@@ -261,10 +311,10 @@ __global__ void __launch_bounds__(256) k_adj_top(Grid g, const float *__restrict
                                                  const float *__restrict__ mx, const float *__restrict__ my,
                                                  const float *__restrict__ X, float alpha,
                                                  const float *__restrict__ E, float beta, float *T, AdjPml pm) {
-  const int i = blockIdx.x * 64 + (int)threadIdx.x + 3, j = blockIdx.y * 4 + (int)threadIdx.y + 3;
+  const int i = blockIdx.x * kTileW + (int)threadIdx.x, j = blockIdx.y * 4 + (int)threadIdx.y + 3;
   const int nk2 = g.nk2;
   const int k = nk2 - (int)blockIdx.z;  /* planes nk2, nk2-1, nk2-2, nk2-3 */
-  if (i >= g.ni + 3 || j >= g.nj + 3 || k < 3) return;
+  if (i < 3 || i >= g.ni + 3 || j >= g.nj + 3 || k < 3) return;
   if (pm.fs.nfault > 0 && fault_column(pm.fs, i, j + (long)k * g.ny)) return;
   const long sc = g.sicmp, sy = g.siy, sz = g.siz;
   const long p = i + j * sy + (long)k * sz;
@@ -279,39 +329,41 @@ __global__ void __launch_bounds__(256) k_adj_top(Grid g, const float *__restrict
     /* timg: h_c = s/J(p) sum_taps coef J(q) (xi_d(q) . T_c(q)), odd image above the surface */
     const int n_free = nk2 - k - fzo;
     const float sj = s / met[p];
-#pragma unroll 1
-    for (int cc = 0; cc < 3; cc++) {
-      const float w = c[cc] * sj;
+    /* the taps' places and their coef J xi_d, for all three components at
+       once; a tap off the grid weighs zero and is placed at the point itself */
+    long dq[3][5];
+    float u[3][5][3];
+#pragma unroll
+    for (int d = 0; d < 3; d++)
 #pragma unroll
       for (int n = 0; n < 5; n++) {
-        {
-          const int ti = i + fxo + n;
-          if (phys(g, ti, j, k)) {
-            const long q = p + fxo + n;
-            const float u = w * tap_coef<ID>(n) * met[q];
-#pragma unroll
-            for (int a = 0; a < 3; a++) atomicAdd(T + tf[cc][a] * sc + q, u * met[(1 + a) * sc + q]);
-          }
+        int off = d == 0 ? fxo + n : (d == 1 ? fyo + n : fzo + n);
+        float w = d == 0 ? tap_coef<ID>(n) : (d == 1 ? tap_coef<JD>(n) : tap_coef<KD>(n));
+        if (d == 2 && n >= n_free) {
+          if (n == n_free) w = 0.0f;  /* the surface itself */
+          off -= 2 * (n - n_free);
+          w = -w;
         }
-        {
-          const int tj = j + fyo + n;
-          if (phys(g, i, tj, k)) {
-            const long q = p + (long)(fyo + n) * sy;
-            const float u = w * tap_coef<JD>(n) * met[q];
+        const bool in = phys(g, i + (d == 0 ? off : 0), j + (d == 1 ? off : 0), k + (d == 2 ? off : 0)) && w != 0.0f;
+        dq[d][n] = in ? off * (d == 0 ? 1 : (d == 1 ? sy : sz)) : 0;
+        const long q = p + dq[d][n];
+        const float jw = in ? w * sj * met[q] : 0.0f;
 #pragma unroll
-            for (int a = 0; a < 3; a++) atomicAdd(T + tf[cc][a] * sc + q, u * met[(4 + a) * sc + q]);
-          }
-        }
-        if (n == n_free) continue;
-        const int dz = n < n_free ? fzo + n : fzo + n - 2 * (n - n_free);
-        const float sign = n < n_free ? 1.0f : -1.0f;
-        if (phys(g, i, j, k + dz)) {
-          const long q = p + (long)dz * sz;
-          const float u = sign * w * tap_coef<KD>(n) * met[q];
-#pragma unroll
-          for (int a = 0; a < 3; a++) atomicAdd(T + tf[cc][a] * sc + q, u * met[(7 + a) * sc + q]);
-        }
+        for (int a = 0; a < 3; a++) u[d][n][a] = jw * met[(1 + 3 * d + a) * sc + q];
       }
+#pragma unroll 1
+    for (int cc = 0; cc < 3; cc++) {
+      const float w = c[cc];
+      const bool bad = !(fabsf(w) < __builtin_inff());  /* not finite: also where u is zero */
+      float *T0 = T + p;
+#pragma unroll
+      for (int d = 0; d < 3; d++)
+#pragma unroll
+        for (int n = 0; n < 5; n++) {
+#pragma unroll
+          for (int a = 0; a < 3; a++)
+            if (u[d][n][a] != 0.0f || bad) atomicAdd(T0 + tf[cc][a] * sc + dq[d][n], w * u[d][n][a]);
+        }
     }
   }
 
@@ -422,7 +474,7 @@ template <int ID, int JD, int KD>
 static void adj_top_dir(int mode, const Grid &g, const float *met, const float *lam, const float *mu,
                         const float *slw, const float *mx, const float *my, const float *X, float alpha,
                         const float *E, float beta, float *T, const AdjPml &pm, hipStream_t st) {
-  dim3 blk(64, 4, 1), grd((g.ni + 63) / 64, (g.nj + 3) / 4, g.nk < 4 ? g.nk : 4);
+  dim3 blk(kTileW, 4, 1), grd(tiles_x(g), (g.nj + 3) / 4, g.nk < 4 ? g.nk : 4);
   switch (mode) {
     case 3:
       hipLaunchKernelGGL((k_adj_top<ID, JD, KD, 3>), grd, blk, 0, st, g, met, lam, mu, slw, mx, my, X, alpha, E,
@@ -476,7 +528,7 @@ __global__ void k_adj_inject(const long *__restrict__ term, const float *__restr
 void launch_adj_prep(int mode, const Grid &g, const float *lam, const float *mu, const float *slw, const float *X,
                      float alpha, const float *E, float beta, float *SG, const AdjPml &pm, int isfree, int kdir,
                      hipStream_t st) {
-  dim3 blk(64, 4, 1), grd((g.ni + 63) / 64, (g.nj + 3) / 4, g.nk);
+  dim3 blk(kTileW, 4, 1), grd(tiles_x(g), (g.nj + 3) / 4, g.nk);
   switch (mode) {
     case 3:
       hipLaunchKernelGGL(k_adj_prep<3>, grd, blk, 0, st, g, lam, mu, slw, X, alpha, E, beta, SG, pm, isfree, kdir);
@@ -496,7 +548,7 @@ void launch_adj_prep(int mode, const Grid &g, const float *lam, const float *mu,
 template <int ID, int JD, int KD, bool VC>
 static void adj_stage_dir(int mode, const Grid &g, const float *met, const float *SG, const float *E, float *A,
                           float *B, float *P, const AdjPml &pm, hipStream_t st) {
-  dim3 blk(64, 4, 1), grd((g.ni + 63) / 64, (g.nj + 3) / 4, g.nk);
+  dim3 blk(kTileW, 2, 2), grd(tiles_x(g), (g.nj + 1) / 2, (g.nk + 1) / 2);
   switch (mode) {
     case 3: hipLaunchKernelGGL((k_adj_stage<ID, JD, KD, 3, VC>), grd, blk, 0, st, g, met, SG, E, A, B, P, pm); break;
     case 2: hipLaunchKernelGGL((k_adj_stage<ID, JD, KD, 2, VC>), grd, blk, 0, st, g, met, SG, E, A, B, P, pm); break;
