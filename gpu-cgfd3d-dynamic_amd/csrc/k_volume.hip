@@ -858,12 +858,12 @@ DEVI void top_point(const VolArgs &a, int i, int j, int k, long woff, long poff)
 /* grid z = plane x scenario */
 template <int ID, int JD, int KD, bool VC>
 __global__ void __launch_bounds__(256) k_vol_top(VolArgs a, BatArgs b) {
-  const int ix = blockIdx.x * blockDim.x + threadIdx.x;
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;  /* aligned tiles */
   const int iy = blockIdx.y * blockDim.y + threadIdx.y;
-  if (ix >= a.g.ni || iy >= a.g.nj) return;
+  if (i < 3 || i >= a.g.ni + 3 || iy >= a.g.nj) return;
   const int kz = (int)blockIdx.z % a.nk_run;
   const long sn = b.act[blockIdx.z / a.nk_run];
-  top_point<ID, JD, KD, VC>(a, ix + 3, iy + 3, a.k_lo + kz + 3, sn * b.wstride, sn * b.pstride);
+  top_point<ID, JD, KD, VC>(a, i, iy + 3, a.k_lo + kz + 3, sn * b.wstride, sn * b.pstride);
 }
 
 /* ------------------------------------------------------------------------
@@ -1017,10 +1017,9 @@ static void launch_box_split(int tw, bool sweeps, bool grouped, bool one, const 
 template <int ID, int JD, int KD>
 static void launch_dir(int variant, const VolArgs &a, const BatArgs &b, int top, hipStream_t st, hipStream_t st_pml) {
   dim3 blk(64, 4, 1);
-  dim3 grd((a.g.ni + 63) / 64, (a.g.nj + 3) / 4, a.nk_run);
   dim3 agrd((a.g.ni + 3 + 63) / 64, (a.g.nj + 3) / 4, a.nk_run);  /* aligned tiles */
   if (top) {
-    dim3 tgrd(grd.x, grd.y, (unsigned)(a.nk_run * b.nact));
+    dim3 tgrd(agrd.x, agrd.y, (unsigned)(a.nk_run * b.nact));
     if (a.vcol) hipLaunchKernelGGL((k_vol_top<ID, JD, KD, true>), tgrd, blk, 0, st, a, b);
     else hipLaunchKernelGGL((k_vol_top<ID, JD, KD, false>), tgrd, blk, 0, st, a, b);
     return;
