@@ -51,7 +51,6 @@ constexpr int kOffT1 = 72, kOffHT1 = 93, kOffMT1 = 96, kOffSlip = 99, kOffGrad =
               kOffVsr = 109;
 
 DEVI void aadd(float *p, float v) { atomicAdd(p, v); }
-
 /* transposes of the fd_t.h difference macros: add a * d(op)/d(tap) */
 DEVI void t_mac22(float *p, long s, int f, float a) {
   if (f == 1) { aadd(p + s, a); aadd(p, -a); }
@@ -109,14 +108,18 @@ DEVI void metric_cols(const float *met, long sc, long p, float M[3][3]) {
   M[2][0] = met[3 * sc + p]; M[2][1] = met[6 * sc + p]; M[2][2] = met[9 * sc + p];
 }
 
-/* fault2wave_node (k_fault.hip, transform.cu:331-372) transposed: the
-   adjoint aw of the nine wavefield values written at the plane goes to the
-   split-node state adjoint af (own node; atomic) and to T1 slot 3 */
-DEVI void t_fault2wave(const AdjFaultArgs &a, long pf, long p, const float *aw, float *af, float *aT1) {
-  const long sc = a.g.sicmp, ss = a.g.sslice;
-  float M[3][3];
-  metric_cols(a.met, sc, p, M);
-  const float rj = (float)(1.0 / a.met[p]);
+/* jac and the nine metric entries of a point, metric_cols' order */
+DEVI void load_met(const float *met, long sc, long p, float &jac, float M[3][3]) {
+  jac = met[p];
+  metric_cols(met, sc, p, M);
+}
+
+/* fault2wave_node (k_fault.hip, transform.cu:331-372) transposed: from the
+   adjoint aw of the nine wavefield values written at the plane, t[c] for T1
+   slot 3 (t[c][0]) and the split-node tractions 2 and 3 (half of t[c][1] and
+   t[c][2] to each side). M: metric_cols of the point (inverted in place) */
+DEVI void f2w_adj(const AdjFaultArgs &a, float jac, float M[3][3], const float *aw, float t[3][3]) {
+  const float rj = (float)(1.0 / jac);
   inv3(M);
   float aS[3][3];
   aS[0][0] = aw[TXX];
@@ -127,82 +130,110 @@ DEVI void t_fault2wave(const AdjFaultArgs &a, long pf, long p, const float *aw, 
   aS[0][2] = aS[2][0] = 0.5f * axz;
   aS[1][2] = aS[2][1] = 0.5f * ayz;
 #pragma unroll
-  for (int c = 0; c < 3; c++) {
-    float t[3];
+  for (int c = 0; c < 3; c++)
 #pragma unroll
-    for (int k = 0; k < 3; k++) t[k] = rj * (aS[c][0] * M[k][0] + aS[c][1] * M[k][1] + aS[c][2] * M[k][2]);
-    aT1[(long)(7 * c + 3) * ss + pf] += t[0];
+    for (int k = 0; k < 3; k++) t[c][k] = rj * (aS[c][0] * M[k][0] + aS[c][1] * M[k][1] + aS[c][2] * M[k][2]);
+}
+/* its split-node state adjoints (own node; atomic) */
+DEVI void f2w_scatter(const float t[3][3], const float *aw, float *af, long ss, long pf) {
+#pragma unroll
+  for (int c = 0; c < 3; c++)
 #pragma unroll
     for (int m = 0; m < 2; m++) {
-      aadd(af + fidx(3 + c, m, ss) + pf, 0.5f * t[1]);
-      aadd(af + fidx(6 + c, m, ss) + pf, 0.5f * t[2]);
+      aadd(af + fidx(3 + c, m, ss) + pf, 0.5f * t[c][1]);
+      aadd(af + fidx(6 + c, m, ss) + pf, 0.5f * t[c][2]);
       aadd(af + fidx(c, m, ss) + pf, 0.5f * aw[c]);
     }
-  }
 }
 
 DEVI float *adj_block(const AdjFaultArgs &a, int id) { return a.adjf + (long)id * kAdjFaultFloats * a.g.sslice; }
 DEVI float *adj_lev(const AdjFaultArgs &a, float *blk, int l) { return l < 0 ? nullptr : blk + (long)l * 18 * a.g.sslice; }
 
+/* The node kernels: one lane per node, a block of one wavefront (a fault plane
+   is 100 to 3000 wavefronts on 256 CUs, so nothing hides a wait), and every
+   load ahead of the first store or atomic: the vector memory counter is in
+   order, so a load issued after an atomic waits for it as well. Measured at
+   48 x 128 nodes (240 x 100): trial 29.6 -> 11.9 us (44 -> 21), nodes 28.8 ->
+   25.5 (41 -> 38), w2f 11.9 -> 5.0 (21 -> 9.7), lev 6.7 -> 4.8 (8.8 -> 5.3),
+   begin 14.2 -> 6.0 (19 -> 16). */
+constexpr int kNodeLanes = 64;
+
 /* ---------------------------------------------------------------------- */
 /* Once per reverse step, before its last stage: the split-node P level is
    cleared (it accumulates over the step); the last stage's hT1/mT1 update,
    Slip += |V_s| dt and the fault2wave onto the end level are transposed. */
-__global__ void __launch_bounds__(256) k_adjf_begin(AdjFaultArgs a) {
-  const int iy = blockIdx.x * blockDim.x + threadIdx.x, iz = blockIdx.y * blockDim.y + threadIdx.y;
-  if (iy >= a.g.nj || iz >= a.g.nk) return;
+__global__ void __launch_bounds__(kNodeLanes) k_adjf_begin(AdjFaultArgs a) {
+  const int iy = blockIdx.x * kNodeLanes + threadIdx.x, iz = blockIdx.y;
+  if (iy >= a.g.nj) return;
   const int id = blockIdx.z;
   const FaultDev &F = a.ftab[id];
   const long ss = a.g.sslice, sc = a.g.sicmp;
   const long pf = (iy + 3) + (long)(iz + 3) * a.g.ny;
   float *blk = adj_block(a, id);
   float *fP = adj_lev(a, blk, a.lp), *fE = adj_lev(a, blk, a.le);
+  if (F.united[pf] != 0) {
 #pragma unroll
-  for (int q = 0; q < 18; q++) fP[q * ss + pf] = 0.0f;
-  if (F.united[pf] != 0) return;
+    for (int q = 0; q < 18; q++) fP[q * ss + pf] = 0.0f;
+    return;
+  }
   float *aT1 = blk + kOffT1 * ss, *aH = blk + kOffHT1 * ss, *aM = blk + kOffMT1 * ss;
   const float dt = a.dt;
+  const long p0 = F.i0 + (long)(iy + 3) * a.g.siy + (long)(iz + 3) * a.g.siz;
+  const float *tp = a.tape + ((long)id * a.tape_nt + a.n) * kTapeFloats * ss + pf;
+  float *vr = blk + kOffVsr * ss + pf;
+  /* loads */
+  float h[3], m1[3], t3[3], dV[3], s1[3], s2[3], aw[9], jac, M[3][3];
 #pragma unroll
   for (int c = 0; c < 3; c++) {
-    const float h = aH[c * ss + pf] / dt;
-    aT1[(long)(7 * c + 3) * ss + pf] += h + aM[c * ss + pf];
-    aM[c * ss + pf] = -h;
-    aH[c * ss + pf] = 0.0f;
+    h[c] = aH[c * ss + pf];
+    m1[c] = aM[c * ss + pf];
+    t3[c] = aT1[(long)(7 * c + 3) * ss + pf];
+    dV[c] = tp[(13 + c) * ss];
+    s1[c] = F.vs[c * ss + pf];
+    s2[c] = F.vs[(3 + c) * ss + pf];
   }
+  const float vr0 = vr[0], vr1 = vr[ss], vr2 = vr[2 * ss];
+  const float as0 = blk[kOffSlip * ss + pf], as1 = blk[kOffSlip12 * ss + pf], as2 = blk[(kOffSlip12 + 1) * ss + pf];
+#pragma unroll
+  for (int f = 0; f < 9; f++) aw[f] = a.wE[f * sc + p0];
+  load_met(a.met, sc, p0, jac, M);
+
   /* Vs1, Vs2 = projections of the velocity jump, Vs = |(Vs1, Vs2)|;
      Slip += Vs dt, Slip1 += Vs1 dt, Slip2 += Vs2 dt; plus the receiver
      residuals of Vs, Vs1, Vs2 of this step */
-  const float *tp = a.tape + ((long)id * a.tape_nt + a.n) * kTapeFloats * ss + pf;
-  float dV[3] = {tp[13 * ss], tp[14 * ss], tp[15 * ss]};
-  const float s1[3] = {F.vs[pf], F.vs[ss + pf], F.vs[2 * ss + pf]};
-  const float s2[3] = {F.vs[3 * ss + pf], F.vs[4 * ss + pf], F.vs[5 * ss + pf]};
   const float Vs1 = dV[0] * s1[0] + dV[1] * s1[1] + dV[2] * s1[2];
   const float Vs2 = dV[0] * s2[0] + dV[1] * s2[1] + dV[2] * s2[2];
   const float Vs = sqrtf(Vs2 * Vs2 + Vs1 * Vs1);
-  float *vr = blk + kOffVsr * ss + pf;
-  const float aVs = vr[0] + blk[kOffSlip * ss + pf] * dt;
-  float aV1 = vr[ss] + blk[kOffSlip12 * ss + pf] * dt;
-  float aV2 = vr[2 * ss] + blk[(kOffSlip12 + 1) * ss + pf] * dt;
-  vr[0] = vr[ss] = vr[2 * ss] = 0.0f;
+  const float aVs = vr0 + as0 * dt;
+  float aV1 = vr1 + as1 * dt;
+  float aV2 = vr2 + as2 * dt;
   if (Vs > 0.0f) {
     aV1 += aVs * Vs1 / Vs;
     aV2 += aVs * Vs2 / Vs;
   }
+  /* fault2wave onto the end level */
+  float t[3][3];
+  f2w_adj(a, jac, M, aw, t);
+
+#pragma unroll
+  for (int q = 0; q < 18; q++) fP[q * ss + pf] = 0.0f;
+  vr[0] = vr[ss] = vr[2 * ss] = 0.0f;
+#pragma unroll
+  for (int c = 0; c < 3; c++) {
+    const float hd = h[c] / dt;
+    aT1[(long)(7 * c + 3) * ss + pf] = t3[c] + (hd + m1[c]) + t[c][0];
+    aM[c * ss + pf] = -hd;
+    aH[c * ss + pf] = 0.0f;
+  }
+#pragma unroll
+  for (int f = 0; f < 9; f++) a.wE[f * sc + p0] = 0.0f;
 #pragma unroll
   for (int c = 0; c < 3; c++) {
     const float g = aV1 * s1[c] + aV2 * s2[c];
     aadd(fE + fidx(c, 1, ss) + pf, g);
     aadd(fE + fidx(c, 0, ss) + pf, -g);
   }
-  /* fault2wave onto the end level */
-  const long p0 = F.i0 + (long)(iy + 3) * a.g.siy + (long)(iz + 3) * a.g.siz;
-  float aw[9];
-#pragma unroll
-  for (int f = 0; f < 9; f++) {
-    aw[f] = a.wE[f * sc + p0];
-    a.wE[f * sc + p0] = 0.0f;
-  }
-  t_fault2wave(a, pf, p0, aw, fE, aT1);
+  f2w_scatter(t, aw, fE, ss, pf);
 }
 
 /* fault-receiver residuals of one sample (the outputs after the step being
@@ -231,20 +262,28 @@ __global__ void k_adjf_receivers(AdjFaultArgs a, const int *rec, const float *fa
    wavefield's, k_adjoint.hip): the stage input's adjoint level starts from
    zero (stage 0: P accumulates) */
 template <int MODE>
-__global__ void __launch_bounds__(256) k_adjf_lev(AdjFaultArgs a) {
-  const int iy = blockIdx.x * blockDim.x + threadIdx.x, iz = blockIdx.y * blockDim.y + threadIdx.y;
-  if (iy >= a.g.nj || iz >= a.g.nk) return;
+__global__ void __launch_bounds__(kNodeLanes) k_adjf_lev(AdjFaultArgs a) {
+  const int iy = blockIdx.x * kNodeLanes + threadIdx.x, iz = blockIdx.y;
+  if (iy >= a.g.nj) return;
   const long ss = a.g.sslice;
   const long pf = (iy + 3) + (long)(iz + 3) * a.g.ny;
   float *blk = adj_block(a, blockIdx.z);
-  float *E = adj_lev(a, blk, a.le), *A = adj_lev(a, blk, 1), *B = adj_lev(a, blk, 2), *P = adj_lev(a, blk, a.lp);
+  const float *E = adj_lev(a, blk, a.le);
+  float *A = adj_lev(a, blk, 1), *B = adj_lev(a, blk, 2), *P = adj_lev(a, blk, a.lp);
+  float pv[18];
+  if (MODE != 3) {
+#pragma unroll
+    for (int q = 0; q < 18; q++) {
+      const long o = q * ss + pf;
+      pv[q] = P[o] + (MODE == 2 ? E[o] + A[o] : (MODE == 1 ? B[o] : A[o]));
+    }
+  }
 #pragma unroll
   for (int q = 0; q < 18; q++) {
     const long o = q * ss + pf;
-    if (MODE == 3) A[o] = 0.0f;
-    else if (MODE == 2) { P[o] += E[o] + A[o]; B[o] = 0.0f; }
-    else if (MODE == 1) { P[o] += B[o]; A[o] = 0.0f; }
-    else P[o] += A[o];
+    if (MODE != 3) P[o] = pv[q];
+    if (MODE == 3 || MODE == 1) A[o] = 0.0f;
+    if (MODE == 2) B[o] = 0.0f;
   }
 }
 
@@ -428,9 +467,9 @@ __global__ void __launch_bounds__(256) k_adjf_cols(AdjFaultArgs a) {
 /* ---------------------------------------------------------------------- */
 /* fault_nodes (k_fault.hip) transposed: one lane per node */
 template <int IDIR>
-__global__ void __launch_bounds__(256) k_adjf_nodes(AdjFaultArgs a) {
-  const int iy = blockIdx.x * blockDim.x + threadIdx.x, iz = blockIdx.y * blockDim.y + threadIdx.y;
-  if (iy >= a.g.nj || iz >= a.g.nk) return;
+__global__ void __launch_bounds__(kNodeLanes) k_adjf_nodes(AdjFaultArgs a) {
+  const int iy = blockIdx.x * kNodeLanes + threadIdx.x, iz = blockIdx.y;
+  if (iy >= a.g.nj) return;
   const int id = blockIdx.z;
   const FaultDev &F = a.ftab[id];
   const long ss = a.g.sslice, sc = a.g.sicmp, ny = a.g.ny, sy = a.g.siy, sz = a.g.siz;
@@ -453,6 +492,17 @@ __global__ void __launch_bounds__(256) k_adjf_nodes(AdjFaultArgs a) {
       const long o = fidx(c, mside, ss) + pf;
       r[mside][c] = a.cb * aE[o] + (aX ? a.ca * aX[o] : 0.0f);
     }
+  const float *met = a.met;
+  float *aH = blk + kOffHT1 * ss;
+  const float jac = met[p0], rho[2] = {F.rho_f[pf], F.rho_f[ss + pf]};
+  const bool fgrid = F.faultgrid[pf] == 1;
+  float T1[3][7], h1[3];
+#pragma unroll
+  for (int c = 0; c < 3; c++) {
+    h1[c] = aH[c * ss + pf];
+#pragma unroll
+    for (int t = 0; t < 7; t++) T1[c][t] = aT1[(long)(7 * c + t) * ss + pf];
+  }
   const long ms = ss, mq = 9 * ss;
   /* traction rates fhT2/fhT3 = D (DxV, DyV, DzV) */
   float aDx[2][3] = {}, aDy[2][3] = {}, aDz[2][3] = {};
@@ -547,24 +597,21 @@ __global__ void __launch_bounds__(256) k_adjf_nodes(AdjFaultArgs a) {
       if (ry == 1) t_mac22(q, 1, jdir, aDy[mside][c]);
       else t_macdrp(q, 1, jdir, aDy[mside][c]);
     }
-  if (F.faultgrid[pf] == 1) {
-    float *aH = blk + kOffHT1 * ss;
+  if (fgrid)
 #pragma unroll
-    for (int c = 0; c < 3; c++) aH[c * ss + pf] += aDt[c];
-  }
+    for (int c = 0; c < 3; c++) aH[c * ss + pf] = h1[c] + aDt[c];
   /* split-node velocity rates from T1 and the traction differences */
-  const float *met = a.met;
-#pragma unroll 1
+#pragma unroll
   for (int mside = 0; mside < 2; mside++) {
-    const float rrhojac = (float)(1.0 / (F.rho_f[mside * ss + pf] * met[p0]));
-#pragma unroll 1
+    const float rrhojac = (float)(1.0 / (rho[mside] * jac));
+#pragma unroll
     for (int c = 0; c < 3; c++) {
       const float g = r[mside][c] * rrhojac;
-      float *t = aT1 + (long)c * 7 * ss + pf;
+      float *t = T1[c];
       if (mside == 0) {
-        t[3 * ss] += (float)kA0 * g; t[2 * ss] -= (float)kA1 * g; t[ss] -= (float)kA2 * g; t[0] -= (float)kA3 * g;
+        t[3] += (float)kA0 * g; t[2] -= (float)kA1 * g; t[1] -= (float)kA2 * g; t[0] -= (float)kA3 * g;
       } else {
-        t[3 * ss] -= (float)kA0 * g; t[4 * ss] += (float)kA1 * g; t[5 * ss] += (float)kA2 * g; t[6 * ss] += (float)kA3 * g;
+        t[3] -= (float)kA0 * g; t[4] += (float)kA1 * g; t[5] += (float)kA2 * g; t[6] += (float)kA3 * g;
       }
       float *p2 = aC + fidx(3 + c, mside, ss) + pf, *p3 = aC + fidx(6 + c, mside, ss) + pf;
       if (ry == 1) t_mac22(p2, 1, jdir, g);
@@ -574,14 +621,18 @@ __global__ void __launch_bounds__(256) k_adjf_nodes(AdjFaultArgs a) {
       else if (rz == 0) t_macdrp(p3, ny, kdir, g);
     }
   }
+#pragma unroll
+  for (int c = 0; c < 3; c++)
+#pragma unroll
+    for (int t = 0; t < 7; t++) aT1[(long)(7 * c + t) * ss + pf] = T1[c][t];
 }
 
 /* ---------------------------------------------------------------------- */
 /* trial (k_fault.hip, trial_slipweakening.cu:91-388) and trial_t1
    transposed, with the parameter gradients; one lane per split node */
-__global__ void __launch_bounds__(128) k_adjf_trial(AdjFaultArgs a) {
-  const int iy = blockIdx.x * blockDim.x + threadIdx.x, iz = blockIdx.y * blockDim.y + threadIdx.y;
-  if (iy >= a.g.nj || iz >= a.g.nk) return;
+__global__ void __launch_bounds__(kNodeLanes) k_adjf_trial(AdjFaultArgs a) {
+  const int iy = blockIdx.x * kNodeLanes + threadIdx.x, iz = blockIdx.y;
+  if (iy >= a.g.nj) return;
   const int id = blockIdx.z;
   const FaultDev &F = a.ftab[id];
   const long ss = a.g.sslice, sc = a.g.sicmp, ny = a.g.ny;
@@ -596,34 +647,49 @@ __global__ void __launch_bounds__(128) k_adjf_trial(AdjFaultArgs a) {
   float *blk = adj_block(a, id);
   float *aT1 = blk + kOffT1 * ss, *aC = adj_lev(a, blk, a.lc), *aP = adj_lev(a, blk, a.lp);
   float *gr = blk + kOffGrad * ss;
+  float *W = a.wT;
 
-  /* fault2wave onto the stage input at the plane */
-  {
-    float aw[9];
+  /* loads: the plane and its metric, T1, the tape and parameters, and the
+     three stress columns on either side with their metric rows */
+  float aw[9], jac0, M[3][3], T1[3][7], w6[6][6], m4[6][4], g7[7];
 #pragma unroll
-    for (int f = 0; f < 9; f++) {
-      aw[f] = a.wT[f * sc + p0];
-      a.wT[f * sc + p0] = 0.0f;
-    }
-    t_fault2wave(a, pf, p0, aw, aC, aT1);
+  for (int f = 0; f < 9; f++) aw[f] = W[f * sc + p0];
+  load_met(met, sc, p0, jac0, M);
+#pragma unroll
+  for (int c = 0; c < 3; c++)
+#pragma unroll
+    for (int t = 0; t < 7; t++) T1[c][t] = aT1[(long)(7 * c + t) * ss + pf];
+  const float *tp = a.tape + ((long)id * a.tape_nt + a.n) * kTapeFloats * ss + pf;
+  const float Trial[3] = {tp[(3 * a.istage) * ss], tp[(3 * a.istage + 1) * ss], tp[(3 * a.istage + 2) * ss]};
+  const float Slip = tp[12 * ss];
+  const float T0[3] = {F.T0[pf], F.T0[ss + pf], F.T0[2 * ss + pf]};
+  const float mus = F.fric[pf], mud = F.fric[ss + pf], Dc = F.fric[2 * ss + pf], C0 = F.fric[3 * ss + pf];
+  const float rho0 = F.rho_f[pf], rho1 = F.rho_f[ss + pf];
+#pragma unroll
+  for (int q = 0; q < 7; q++) g7[q] = gr[q * ss + pf];
+  const float aSlip = blk[kOffSlip * ss + pf];
+#pragma unroll
+  for (int l = 0; l < 6; l++) {
+    const long q = p0 + (l < 3 ? l - 3 : l - 2);
+#pragma unroll
+    for (int f = 0; f < 6; f++) w6[l][f] = W[(TXX + f) * sc + q];
+#pragma unroll
+    for (int f = 0; f < 4; f++) m4[l][f] = met[f * sc + q];
   }
+
+  float vn[3] = {M[0][0], M[1][0], M[2][0]};
+  /* fault2wave onto the stage input at the plane */
+  float tw[3][3];
+  f2w_adj(a, jac0, M, aw, tw);
 
   /* friction on the taped branch */
-  const float *tp = a.tape + ((long)id * a.tape_nt + a.n) * kTapeFloats * ss + pf;
-  float Trial[3] = {tp[(3 * a.istage) * ss], tp[(3 * a.istage + 1) * ss], tp[(3 * a.istage + 2) * ss]};
-  const float Slip = tp[12 * ss];
   float at[3];
 #pragma unroll
-  for (int c = 0; c < 3; c++) {
-    at[c] = aT1[(long)(7 * c + 3) * ss + pf];
-    aT1[(long)(7 * c + 3) * ss + pf] = 0.0f;
-  }
-  float vn[3] = {met[sc + p0], met[2 * sc + p0], met[3 * sc + p0]};
+  for (int c = 0; c < 3; c++) at[c] = T1[c][3] + tw[c][0];
   const float vn0 = norm3(vn);
-  const float jacvec = met[p0] * vn0;
+  const float jacvec = jac0 * vn0;
 #pragma unroll
   for (int c = 0; c < 3; c++) vn[c] /= vn0;
-  const float T0[3] = {F.T0[pf], F.T0[ss + pf], F.T0[2 * ss + pf]};
   float TL[3], Ts[3];
 #pragma unroll
   for (int c = 0; c < 3; c++) TL[c] = Trial[c] / jacvec + T0[c];
@@ -633,7 +699,6 @@ __global__ void __launch_bounds__(128) k_adjf_trial(AdjFaultArgs a) {
   const float Ts0 = norm3(Ts);
   const bool open = Tn0 >= 0.0f;
   const float Tau_n = open ? 0.0f : Tn0;
-  const float mus = F.fric[pf], mud = F.fric[ss + pf], Dc = F.fric[2 * ss + pf], C0 = F.fric[3 * ss + pf];
   const bool weak = Slip <= Dc;
   const float fr = weak ? mus - (mus - mud) * Slip / Dc : mud;
   const float Tau_c = -fr * Tau_n + C0;
@@ -668,14 +733,14 @@ __global__ void __launch_bounds__(128) k_adjf_trial(AdjFaultArgs a) {
     /* Tau_c = -fr Tau_n + C0 */
     const float afr = -aTau_c * Tau_n;
     aTau_n += -fr * aTau_c;
-    gr[3 * ss + pf] += aTau_c;
+    gr[3 * ss + pf] = g7[3] + aTau_c;
     if (weak) {
-      gr[pf] += afr * (1.0f - Slip / Dc);
-      gr[ss + pf] += afr * (Slip / Dc);
-      gr[2 * ss + pf] += afr * (mus - mud) * Slip / (Dc * Dc);
-      blk[kOffSlip * ss + pf] += -afr * (mus - mud) / Dc;
+      gr[pf] = g7[0] + afr * (1.0f - Slip / Dc);
+      gr[ss + pf] = g7[1] + afr * (Slip / Dc);
+      gr[2 * ss + pf] = g7[2] + afr * (mus - mud) * Slip / (Dc * Dc);
+      blk[kOffSlip * ss + pf] = aSlip - afr * (mus - mud) / Dc;
     } else {
-      gr[ss + pf] += afr;
+      gr[ss + pf] = g7[1] + afr;
     }
     float aTn0 = open ? 0.0f : aTau_n;
     if (Ts0 > 0.0f)
@@ -689,62 +754,74 @@ __global__ void __launch_bounds__(128) k_adjf_trial(AdjFaultArgs a) {
 #pragma unroll
     for (int c = 0; c < 3; c++) {
       aTrial[c] = aTL[c] / jacvec;
-      gr[(4 + c) * ss + pf] += aTL[c] + aT0[c];
+      gr[(4 + c) * ss + pf] = g7[4 + c] + (aTL[c] + aT0[c]);
     }
   }
 
   /* Trial = 2 (M0 M1 dV / dt + M0 R1 - M1 R0) / (a0 (M0 + M1)) */
-  const float jac0 = met[p0];
-  const float M0 = (float)(0.5 * jac0 * F.rho_f[pf]), M1 = (float)(0.5 * jac0 * F.rho_f[ss + pf]);
+  const float M0 = (float)(0.5 * jac0 * rho0), M1 = (float)(0.5 * jac0 * rho1);
   const float den = (float)(2.0 / (kA0 * (M0 + M1)));
-#pragma unroll 1
+  float ad[2][3], adv[3];
+#pragma unroll
   for (int c = 0; c < 3; c++) {
     const float g = aTrial[c] * den;
-    const float adv = g * M0 * M1 / a.dt;
-    aadd(aP + fidx(c, 1, ss) + pf, adv);
-    aadd(aP + fidx(c, 0, ss) + pf, -adv);
-#pragma unroll 1
+    adv[c] = g * M0 * M1 / a.dt;
+#pragma unroll
     for (int mside = 0; mside < 2; mside++) {
+      const int sd = 2 * mside - 1;
       const float aR = mside ? g * M0 : -g * M1;
-      const float ar = 0.5f * (float)(2 * mside - 1) * aR, ad = 0.5f * aR;
-      float *t = aT1 + (long)c * 7 * ss + pf;
-      t[(3 + (2 * mside - 1)) * ss] += (float)kA1 * ar;
-      t[(3 + 2 * (2 * mside - 1)) * ss] += (float)kA2 * ar;
-      t[(3 + 3 * (2 * mside - 1)) * ss] += (float)kA3 * ar;
-      float *p2 = aC + fidx(3 + c, mside, ss) + pf, *p3 = aC + fidx(6 + c, mside, ss) + pf;
-      if (ry == 1) t_mac22(p2, 1, jdir, ad);
-      else if (ry == 0) t_macdrp(p2, 1, jdir, ad);
-      if (a.isfree == 1 && km <= 3) t_dz_free_image(p3, ny, n_free, kdir, ad);
-      else if (rz == 1) t_mac22(p3, ny, kdir, ad);
-      else if (rz == 0) t_macdrp(p3, ny, kdir, ad);
+      const float ar = 0.5f * (float)sd * aR;
+      ad[mside][c] = 0.5f * aR;
+      T1[c][3 + sd] += (float)kA1 * ar;
+      T1[c][3 + 2 * sd] += (float)kA2 * ar;
+      T1[c][3 + 3 * sd] += (float)kA3 * ar;
     }
   }
 
   /* traction columns T1 slots 0-2 / 4-6 from the stress (trial_t1) */
-#pragma unroll 1
-  for (int mside = 0; mside < 2; mside++)
-#pragma unroll 1
-    for (int l = 1; l <= 3; l++) {
-      const long slot = 3 + (2 * mside - 1) * l;
-      const long q = F.i0 + (2 * mside - 1) * l + row;
-      const float jl = met[q], x1 = met[sc + q], x2 = met[2 * sc + q], x3 = met[3 * sc + q];
-      float *t = aT1 + slot * ss + pf;
-      const float a0 = jl * t[0], a1 = jl * t[7 * ss], a2 = jl * t[14 * ss];
-      t[0] = t[7 * ss] = t[14 * ss] = 0.0f;
-      float *W = a.wT;
-      W[TXX * sc + q] += x1 * a0;
-      W[TXY * sc + q] += x2 * a0 + x1 * a1;
-      W[TXZ * sc + q] += x3 * a0 + x1 * a2;
-      W[TYY * sc + q] += x2 * a1;
-      W[TYZ * sc + q] += x3 * a1 + x2 * a2;
-      W[TZZ * sc + q] += x3 * a2;
+#pragma unroll
+  for (int l = 0; l < 6; l++) {
+    const int slot = l < 3 ? l : l + 1;
+    const long q = p0 + (slot - 3);
+    const float jl = m4[l][0], x1 = m4[l][1], x2 = m4[l][2], x3 = m4[l][3];
+    const float a0 = jl * T1[0][slot], a1 = jl * T1[1][slot], a2 = jl * T1[2][slot];
+    const float *w = w6[l];
+    W[TXX * sc + q] = w[TXX - TXX] + x1 * a0;
+    W[TXY * sc + q] = w[TXY - TXX] + (x2 * a0 + x1 * a1);
+    W[TXZ * sc + q] = w[TXZ - TXX] + (x3 * a0 + x1 * a2);
+    W[TYY * sc + q] = w[TYY - TXX] + x2 * a1;
+    W[TYZ * sc + q] = w[TYZ - TXX] + (x3 * a1 + x2 * a2);
+    W[TZZ * sc + q] = w[TZZ - TXX] + x3 * a2;
+  }
+#pragma unroll
+  for (int f = 0; f < 9; f++) W[f * sc + p0] = 0.0f;
+#pragma unroll
+  for (int c = 0; c < 3; c++)
+#pragma unroll
+    for (int t = 0; t < 7; t++) aT1[(long)(7 * c + t) * ss + pf] = 0.0f;
+
+  f2w_scatter(tw, aw, aC, ss, pf);
+#pragma unroll
+  for (int c = 0; c < 3; c++) {
+    aadd(aP + fidx(c, 1, ss) + pf, adv[c]);
+    aadd(aP + fidx(c, 0, ss) + pf, -adv[c]);
+#pragma unroll
+    for (int mside = 0; mside < 2; mside++) {
+      float *p2 = aC + fidx(3 + c, mside, ss) + pf, *p3 = aC + fidx(6 + c, mside, ss) + pf;
+      const float g = ad[mside][c];
+      if (ry == 1) t_mac22(p2, 1, jdir, g);
+      else if (ry == 0) t_macdrp(p2, 1, jdir, g);
+      if (a.isfree == 1 && km <= 3) t_dz_free_image(p3, ny, n_free, kdir, g);
+      else if (rz == 1) t_mac22(p3, ny, kdir, g);
+      else if (rz == 0) t_macdrp(p3, ny, kdir, g);
     }
+  }
 }
 
 /* wave2fault (k_fault.hip, transform.cu:100-212) transposed at welded nodes */
-__global__ void __launch_bounds__(256) k_adjf_w2f(AdjFaultArgs a) {
-  const int iy = blockIdx.x * blockDim.x + threadIdx.x, iz = blockIdx.y * blockDim.y + threadIdx.y;
-  if (iy >= a.g.nj || iz >= a.g.nk) return;
+__global__ void __launch_bounds__(kNodeLanes) k_adjf_w2f(AdjFaultArgs a) {
+  const int iy = blockIdx.x * kNodeLanes + threadIdx.x, iz = blockIdx.y;
+  if (iy >= a.g.nj) return;
   const int id = blockIdx.z;
   const FaultDev &F = a.ftab[id];
   const long ss = a.g.sslice, sc = a.g.sicmp;
@@ -753,11 +830,11 @@ __global__ void __launch_bounds__(256) k_adjf_w2f(AdjFaultArgs a) {
   const long p = F.i0 + (long)(iy + 3) * a.g.siy + (long)(iz + 3) * a.g.siz;
   float *blk = adj_block(a, id);
   float *aT1 = blk + kOffT1 * ss, *aC = adj_lev(a, blk, a.lc);
-  float aTr[3][3], aV[3];
+  float *W = a.wT;
+  float aTr[3][3], aV[3], w[9], jac, M[3][3];
 #pragma unroll
   for (int c = 0; c < 3; c++) {
     aTr[c][0] = aT1[(long)(7 * c + 3) * ss + pf];
-    aT1[(long)(7 * c + 3) * ss + pf] = 0.0f;
     aTr[c][1] = aTr[c][2] = aV[c] = 0.0f;
 #pragma unroll
     for (int m = 0; m < 2; m++) {
@@ -766,33 +843,35 @@ __global__ void __launch_bounds__(256) k_adjf_w2f(AdjFaultArgs a) {
       aTr[c][2] += aC[fidx(6 + c, m, ss) + pf];
     }
   }
+  load_met(a.met, sc, p, jac, M);
 #pragma unroll
-  for (int q = 0; q < 18; q++) aC[q * ss + pf] = 0.0f;
-  float M[3][3];
-  metric_cols(a.met, sc, p, M);
-  const float jac = a.met[p];
+  for (int f = 0; f < 9; f++) w[f] = W[f * sc + p];
   float aS[3][3];
 #pragma unroll
   for (int r = 0; r < 3; r++)
 #pragma unroll
     for (int k = 0; k < 3; k++) aS[r][k] = jac * (aTr[r][0] * M[k][0] + aTr[r][1] * M[k][1] + aTr[r][2] * M[k][2]);
-  float *W = a.wT;
 #pragma unroll
-  for (int c = 0; c < 3; c++) W[c * sc + p] += aV[c];
-  W[TXX * sc + p] += aS[0][0];
-  W[TYY * sc + p] += aS[1][1];
-  W[TZZ * sc + p] += aS[2][2];
-  W[TXY * sc + p] += aS[0][1] + aS[1][0];
-  W[TXZ * sc + p] += aS[0][2] + aS[2][0];
-  W[TYZ * sc + p] += aS[1][2] + aS[2][1];
+  for (int c = 0; c < 3; c++) {
+    aT1[(long)(7 * c + 3) * ss + pf] = 0.0f;
+    W[c * sc + p] = w[c] + aV[c];
+  }
+#pragma unroll
+  for (int q = 0; q < 18; q++) aC[q * ss + pf] = 0.0f;
+  W[TXX * sc + p] = w[TXX] + aS[0][0];
+  W[TYY * sc + p] = w[TYY] + aS[1][1];
+  W[TZZ * sc + p] = w[TZZ] + aS[2][2];
+  W[TXY * sc + p] = w[TXY] + (aS[0][1] + aS[1][0]);
+  W[TXZ * sc + p] = w[TXZ] + (aS[0][2] + aS[2][0]);
+  W[TYZ * sc + p] = w[TYZ] + (aS[1][2] + aS[2][1]);
 }
 
 /* ---------------------------------------------------------------------- */
-static dim3 node_grid(const AdjFaultArgs &a) { return dim3((a.g.nj + 63) / 64, (a.g.nk + 3) / 4, a.nfault); }
+static dim3 node_grid(const AdjFaultArgs &a) { return dim3((a.g.nj + kNodeLanes - 1) / kNodeLanes, a.g.nk, a.nfault); }
 
 void launch_adjf_begin(const AdjFaultArgs &a, hipStream_t st) {
   if (a.nfault <= 0) return;
-  hipLaunchKernelGGL(k_adjf_begin, node_grid(a), dim3(64, 4), 0, st, a);
+  hipLaunchKernelGGL(k_adjf_begin, node_grid(a), dim3(kNodeLanes), 0, st, a);
 }
 
 void launch_adjf_receivers(const AdjFaultArgs &a, const int *rec, const float *fac, int nterm, int nrec,
@@ -804,7 +883,7 @@ void launch_adjf_receivers(const AdjFaultArgs &a, const int *rec, const float *f
 
 void launch_adjf_stage_pre(const AdjFaultArgs &a, hipStream_t st) {
   if (a.nfault <= 0) return;
-  const dim3 g = node_grid(a), b(64, 4);
+  const dim3 g = node_grid(a), b(kNodeLanes);
   switch (a.istage) {
     case 3: hipLaunchKernelGGL(k_adjf_lev<3>, g, b, 0, st, a); break;
     case 2: hipLaunchKernelGGL(k_adjf_lev<2>, g, b, 0, st, a); break;
@@ -818,13 +897,13 @@ void launch_adjf_stage_post(const AdjFaultArgs &a, hipStream_t st) {
   const dim3 cg((a.g.nj + kColNodes - 1) / kColNodes, (a.g.nk + 3) / 4, a.nfault), b(64, 4);
   if (a.idir == 1) {
     hipLaunchKernelGGL(k_adjf_cols<1>, cg, b, 0, st, a);
-    hipLaunchKernelGGL(k_adjf_nodes<1>, node_grid(a), b, 0, st, a);
+    hipLaunchKernelGGL(k_adjf_nodes<1>, node_grid(a), dim3(kNodeLanes), 0, st, a);
   } else {
     hipLaunchKernelGGL(k_adjf_cols<0>, cg, b, 0, st, a);
-    hipLaunchKernelGGL(k_adjf_nodes<0>, node_grid(a), b, 0, st, a);
+    hipLaunchKernelGGL(k_adjf_nodes<0>, node_grid(a), dim3(kNodeLanes), 0, st, a);
   }
-  hipLaunchKernelGGL(k_adjf_trial, dim3((a.g.nj + 31) / 32, (a.g.nk + 3) / 4, a.nfault), dim3(32, 4), 0, st, a);
-  hipLaunchKernelGGL(k_adjf_w2f, node_grid(a), b, 0, st, a);
+  hipLaunchKernelGGL(k_adjf_trial, node_grid(a), dim3(kNodeLanes), 0, st, a);
+  hipLaunchKernelGGL(k_adjf_w2f, node_grid(a), dim3(kNodeLanes), 0, st, a);
 }
 
 }  // namespace cgfd
