@@ -131,6 +131,13 @@ struct AdjPml {
   AdjFace f[6];           /* dim-major, side-minor */
   FaultSkip fs;           /* fault columns: their rhs belongs to the fault adjoint */
 };
+/* free surface of the adjoint: the sums the prep leaves for the gather of the
+   top planes, [12][4 planes from the surface down][ny][row], zero off the
+   physical points (null without a free surface), and what forms them */
+struct AdjTop {
+  float *src;
+  const float *met, *mx, *my;
+};
 /* fault part of the adjoint (k_adj_fault.hip): per fault a block of
    kAdjFaultFloats x sslice floats: split-node adjoint levels [4][18] (E, A,
    B, P by index), T1 [21], hT1 [3], mT1 [3], Slip [1], parameter gradients
@@ -159,15 +166,13 @@ void launch_adjf_receivers(const AdjFaultArgs &a, const int *rec, const float *f
 void launch_adjf_stage_pre(const AdjFaultArgs &a, hipStream_t st);
 void launch_adjf_stage_post(const AdjFaultArgs &a, hipStream_t st);
 void launch_adj_prep(int mode, const Grid &g, const float *lam, const float *mu, const float *slw, const float *X,
-                     float alpha, const float *E, float beta, float *SG, const AdjPml &pm, int isfree, int kdir,
+                     float alpha, const float *E, float beta, float *SG, const AdjPml &pm, const AdjTop &top, int kdir,
                      hipStream_t st);
-void launch_adj_top(int mode, int idir, int jdir, int kdir, const Grid &g, const float *met, const float *lam,
-                    const float *mu, const float *slw, const float *mx, const float *my, const float *X, float alpha,
-                    const float *E, float beta, float *T, const AdjPml &pm, hipStream_t st);
-/* vcol: the grid's columns are vertical (the gather reads the xi and eta
-   metric rows' one nonzero term each) */
+/* src: AdjTop's; vcol: the grid's columns are vertical (the gather reads the
+   xi and eta metric rows' one nonzero term each) */
 void launch_adj_stage(int mode, int idir, int jdir, int kdir, const Grid &g, const float *met, const float *SG,
-                      const float *E, float *A, float *B, float *P, const AdjPml &pm, int vcol, hipStream_t st);
+                      const float *E, float *A, float *B, float *P, const AdjPml &pm, const float *src, int vcol,
+                      hipStream_t st);
 void launch_adj_inject(const long *term, const float *fac, int nterm, int nsta, const float *res, int nt, int n,
                        long sicmp, float *P, hipStream_t st);
 void launch_record_stations(const BatArgs &b, const float *w, long sicmp, const long *term, const float *fac,

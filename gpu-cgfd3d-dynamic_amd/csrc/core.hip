@@ -969,8 +969,9 @@ int adj_sweep(cgfd_core *c, int scen, const float *residual, const float *residu
       if (c->pml[dim][side].on) npml += 45 * c->pml[dim][side].n;
   if (!c->adj) {
     if ((rc = c->alloc(&c->adj, (size_t)4 * lv))) return rc;
-    if ((rc = c->alloc(&c->adj_sg, (size_t)9 * sc))) return rc;
-    HIPCHK(hipMemset(c->adj_sg, 0, (size_t)9 * sc * 4));  /* ghost entries stay zero */
+    const size_t nsg = (size_t)9 * sc + (c->isfree ? (size_t)48 * g.siz : 0);  /* S, G; the top-layer sums (AdjTop) */
+    if ((rc = c->alloc(&c->adj_sg, nsg))) return rc;
+    HIPCHK(hipMemset(c->adj_sg, 0, nsg * 4));  /* ghost entries stay zero */
     if (npml > 0 && (rc = c->alloc(&c->adj_pml, (size_t)npml))) return rc;
   }
   const size_t nadjf = (size_t)c->nfault * kAdjFaultFloats * ss;
@@ -1001,6 +1002,7 @@ int adj_sweep(cgfd_core *c, int scen, const float *residual, const float *residu
         off += 45 * f.n;
       }
   }
+  const AdjTop top{c->isfree ? c->adj_sg + 9 * sc : nullptr, c->met, c->matVx2Vz, c->matVy2Vz};
   AdjFaultArgs fa{};
   fa.g = g;
   fa.met = c->met; fa.lam = c->lam; fa.mu = c->mu; fa.slw = c->slw;
@@ -1054,11 +1056,9 @@ int adj_sweep(cgfd_core *c, int scen, const float *residual, const float *residu
         fa.lc = s == 0 ? fa.lp : (s == 2 ? 2 : 1);
         fa.wT = T; fa.wX = X; fa.wE = E;
         launch_adjf_stage_pre(fa, c->st);
-        launch_adj_prep(s, g, c->lam, c->mu, c->slw, X, ca, E, cb, c->adj_sg, pm, c->isfree, kdir, c->st);
-        launch_adj_stage(s, idir, jdir, kdir, g, c->met, c->adj_sg, E, A, B, P, pm, c->vcol_grid && c->vcol_on, c->st);
-        if (c->isfree)
-          launch_adj_top(s, idir, jdir, kdir, g, c->met, c->lam, c->mu, c->slw, c->matVx2Vz, c->matVy2Vz, X, ca, E,
-                         cb, T, pm, c->st);
+        launch_adj_prep(s, g, c->lam, c->mu, c->slw, X, ca, E, cb, c->adj_sg, pm, top, kdir, c->st);
+        launch_adj_stage(s, idir, jdir, kdir, g, c->met, c->adj_sg, E, A, B, P, pm, top.src,
+                         c->vcol_grid && c->vcol_on, c->st);
         launch_adjf_stage_post(fa, c->st);
       }
     }

@@ -34,11 +34,14 @@
  * the stress rhs by Hooke's law on the reduced-order velocity gradient
  * (vlow), and the x/y PML faces add a term through the free-surface
  * matrices at the surface. Transposed: the prep leaves out the base S / G of
- * what was replaced, and k_adj_top scatters the adjoint of timg, vlow and
- * the surface PML term onto the taps (atomic adds; ghosts are not state).
+ * what was replaced and writes, for the points of the top four planes, the
+ * adjoints of timg's momentum sums and of vlow's differences (12 values, the
+ * surface PML term among them); the gather of the top five planes adds their
+ * taps. A scatter of the same sums by atomic adds, one kernel more, took 26
+ * of a stage's 52 us at 50 x 71 x 40: device-scope atomics leave the XCD's L2.
  *
  * Fault columns of split nodes (their rhs comes from the fault kernels) get
- * no S and G here and no top-layer scatter; k_adj_fault.hip transposes them.
+ * no S and G here and no top-layer sums; k_adj_fault.hip transposes them.
  *
  * RK4 (drv_rk_curv_col.cu:329-568) with a = {1/2, 1/2, 1}, b = {1/6, 1/3,
  * 1/3, 1/6}, ca = a dt, cb = b dt, reversed (E = adjoint of the step's
@@ -86,6 +89,63 @@ DEVI long face_idx(const AdjFace &F, int i, int j, int k) {
 constexpr int kTileW = 64;
 static unsigned tiles_x(const Grid &g) { return (unsigned)((g.ni + 3 + kTileW - 1) / kTileW); }
 
+/* entry e of the top-layer sums, plane nk2 - kk */
+DEVI long top_idx(const Grid &g, int e, int kk, int i, int j) { return (long)(e * 4 + kk) * g.siz + i + (long)j * g.siy; }
+
+/* Adjoints of the free-surface replacements' own sums at a point of the top
+   four planes, from its rhs adjoint c: entries 0-2 of timg's sums (the taps'
+   coef J xi_d times these), 3-5, 6-8, 9-11 of vlow's D_x, D_y, D_z of V (z:
+   mac22 / mac24; at the surface D_z is a matrix of D_x and D_y). ax, ay: the
+   surface PML term. */
+DEVI void top_source(const Grid &g, const AdjTop &top, int i, int j, int k, long p, const float *c, float l, float m,
+                     float s, const float *ax, const float *ay, int kdir) {
+  const int kk = g.nk2 - k;
+  const long sc = g.sicmp;
+  float w[3] = {0.0f, 0.0f, 0.0f}, dl[3][3] = {};
+  if (kk <= (kdir ? 3 : 1)) {
+    const float sj = s / top.met[p];
+#pragma unroll
+    for (int cc = 0; cc < 3; cc++) w[cc] = c[cc] * sj;
+  }
+  if (kk <= 2) {
+    const float l2m = (float)(l + 2.0 * m);
+    float gm[3][3];  /* adjoint of the physical gradient dV_c/dx_a */
+    gm[0][0] = l2m * c[TXX] + l * c[TYY] + l * c[TZZ];
+    gm[1][1] = l * c[TXX] + l2m * c[TYY] + l * c[TZZ];
+    gm[2][2] = l * c[TXX] + l * c[TYY] + l2m * c[TZZ];
+    gm[0][1] = gm[1][0] = m * c[TXY];
+    gm[0][2] = gm[2][0] = m * c[TXZ];
+    gm[1][2] = gm[2][1] = m * c[TYZ];
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+      const float e0 = top.met[(1 + 3 * d) * sc + p], e1 = top.met[(2 + 3 * d) * sc + p],
+                  e2 = top.met[(3 + 3 * d) * sc + p];
+#pragma unroll
+      for (int cc = 0; cc < 3; cc++) dl[d][cc] = e0 * gm[cc][0] + e1 * gm[cc][1] + e2 * gm[cc][2];
+    }
+    if (kk == 0) {
+      const long ij = ((long)i + (long)j * g.siy) * 9;
+#pragma unroll
+      for (int cc = 0; cc < 3; cc++) {
+        float bx = ax[cc], by = ay[cc];
+#pragma unroll
+        for (int r = 0; r < 3; r++) {
+          bx += top.mx[ij + 3 * r + cc] * dl[2][r];
+          by += top.my[ij + 3 * r + cc] * dl[2][r];
+        }
+        dl[0][cc] += bx;
+        dl[1][cc] += by;
+      }
+    }
+  }
+#pragma unroll
+  for (int cc = 0; cc < 3; cc++) {
+    top.src[top_idx(g, cc, kk, i, j)] = w[cc];
+#pragma unroll
+    for (int d = 0; d < 3; d++) top.src[top_idx(g, 3 + 3 * d + cc, kk, i, j)] = dl[d][cc];
+  }
+}
+
 /* S and G from c = alpha X + beta E at physical points (X may be null);
    at CFS-PML points also the per-face extra S and G and the auxiliaries'
    reverse stage (MODE as k_adj_stage) */
@@ -93,7 +153,7 @@ template <int MODE>
 __global__ void __launch_bounds__(256) k_adj_prep(Grid g, const float *__restrict__ lam, const float *__restrict__ mu,
                                                   const float *__restrict__ slw, const float *__restrict__ X,
                                                   float alpha, const float *__restrict__ E, float beta,
-                                                  float *__restrict__ SG, AdjPml pm, int isfree, int kdir) {
+                                                  float *__restrict__ SG, AdjPml pm, AdjTop top, int kdir) {
   const int i = blockIdx.x * kTileW + (int)threadIdx.x, j = blockIdx.y * 4 + (int)threadIdx.y + 3;
   const int k = (int)blockIdx.z + 3;
   if (i < 3 || i >= g.ni + 3 || j >= g.nj + 3) return;
@@ -102,6 +162,9 @@ __global__ void __launch_bounds__(256) k_adj_prep(Grid g, const float *__restric
   if (pm.fs.nfault > 0 && fault_column(pm.fs, i, j + (long)k * g.ny)) {
 #pragma unroll
     for (int q = 0; q < kSG; q++) SG[q * sc + p] = 0.0f;
+    if (top.src && g.nk2 - k < 4)
+#pragma unroll
+      for (int q = 0; q < 12; q++) top.src[top_idx(g, q, g.nk2 - k, i, j)] = 0.0f;
     return;
   }
   float c[9];
@@ -110,7 +173,7 @@ __global__ void __launch_bounds__(256) k_adj_prep(Grid g, const float *__restric
   const float l = lam[p], m = mu[p], s = slw[p];
   float o[kSG];
   sg_of(c, l, m, s, o);
-  if (isfree) {
+  if (top.src) {
     /* what timg (velocity rhs) and vlow (stress rhs) replace at the top */
     if (k >= g.nk2 - (kdir ? 3 : 1)) o[0] = o[1] = o[2] = 0.0f;
     if (k >= g.nk2 - 2)
@@ -119,9 +182,9 @@ __global__ void __launch_bounds__(256) k_adj_prep(Grid g, const float *__restric
   }
 #pragma unroll
   for (int q = 0; q < kSG; q++) SG[q * sc + p] = o[q];
-  if (!pm.on) return;
+  float ax[3] = {0.0f, 0.0f, 0.0f}, ay[3] = {0.0f, 0.0f, 0.0f};  /* surface PML term: adjoints of D_x V, D_y V */
 #pragma unroll 1
-  for (int fc = 0; fc < 6; fc++) {
+  for (int fc = 0; pm.on && fc < 6; fc++) {
     const AdjFace &F = pm.f[fc];
     if (!in_face(F, i, j, k)) continue;
     const long ia = face_idx(F, i, j, k), n = F.n;
@@ -156,7 +219,25 @@ __global__ void __launch_bounds__(256) k_adj_prep(Grid g, const float *__restric
     sg_of(dc, l, m, s, o);
 #pragma unroll
     for (int q = 0; q < kSG; q++) F.dsg[q * n + ia] = o[q];
+    if (top.src && k == g.nk2 && fc < 4) {
+      /* the free-surface term of the x/y PML faces: qT from D_dim V through
+         the matrices, added to the stress rhs with (B-1) and to the auxiliary
+         rhs with D (sv_curv_col_el_iso_gpu.cu:1000-1060, :1146-1205) */
+      const float l2m = l + 2.0f * m;
+      const float zx = top.met[7 * sc + p], zy = top.met[8 * sc + p], zz = top.met[9 * sc + p];
+      const float q0 = l2m * zx * dc[TXX] + l * zx * dc[TYY] + l * zx * dc[TZZ] + m * zy * dc[TXY] + m * zz * dc[TXZ];
+      const float q1 = l * zy * dc[TXX] + l2m * zy * dc[TYY] + l * zy * dc[TZZ] + m * zx * dc[TXY] + m * zz * dc[TYZ];
+      const float q2 = l * zz * dc[TXX] + l * zz * dc[TYY] + l2m * zz * dc[TZZ] + m * zx * dc[TXZ] + m * zy * dc[TYZ];
+      const float *X = (F.dim == 0 ? top.mx : top.my) + ((long)i + (long)j * g.siy) * 9;
+#pragma unroll
+      for (int cc = 0; cc < 3; cc++) {
+        const float v = X[cc] * q0 + X[3 + cc] * q1 + X[6 + cc] * q2;
+        if (F.dim == 0) ax[cc] += v;
+        else ay[cc] += v;
+      }
+    }
   }
+  if (top.src && g.nk2 - k < 4) top_source(g, top, i, j, k, p, c, l, m, s, ax, ay, kdir);
 }
 
 template <int DIR>
@@ -253,6 +334,72 @@ DEVI void gather_dir(float *lm, const Grid &g, const float *__restrict__ met, co
   }
 }
 
+/* the top-layer sums (top_source) gathered at a point of the top five planes:
+   the transposes of timg, vlow and the surface PML term, added to lm. Points
+   off the grid hold zeros. */
+template <int ID, int JD, int KD>
+DEVI void gather_top(float *lm, const Grid &g, const float *__restrict__ met, const float *__restrict__ src, int i,
+                     int j, int k, long q) {
+  const long sc = g.sicmp, sy = g.siy;
+  const int kt = g.nk2 - k;
+  constexpr int ox = ID ? -1 : -3, oy = JD ? -1 : -3, oz = KD ? -1 : -3;
+  float M[10];
+#pragma unroll
+  for (int e = 0; e < 10; e++) M[e] = met[e * sc + q];
+  float sx[3] = {0.0f, 0.0f, 0.0f}, sy_[3] = {0.0f, 0.0f, 0.0f}, sz_[3] = {0.0f, 0.0f, 0.0f};
+  if (kt <= oz + 4) {
+#pragma unroll
+    for (int cc = 0; cc < 3; cc++)
+#pragma unroll
+      for (int t = 0; t < 5; t++) {
+        sx[cc] += tap_coef<ID>(t) * src[top_idx(g, cc, kt, i, j) - (ox + t)];
+        sy_[cc] += tap_coef<JD>(t) * src[top_idx(g, cc, kt, i, j) - (oy + t) * sy];
+      }
+  }
+  if (kt <= 2) {
+#pragma unroll
+    for (int cc = 0; cc < 3; cc++)
+#pragma unroll
+      for (int t = 0; t < 5; t++)
+        lm[cc] += tap_coef<ID>(t) * src[top_idx(g, 3 + cc, kt, i, j) - (ox + t)] +
+                  tap_coef<JD>(t) * src[top_idx(g, 6 + cc, kt, i, j) - (oy + t) * sy];
+  }
+  if (kt > 0) {
+    /* a tap of plane ks (nk2 - ks) on this plane, and the one above the
+       surface whose odd image this plane is */
+#pragma unroll
+    for (int ks = 0; ks <= oz + 4; ks++) {
+      const int n1 = ks - kt - oz, n2 = ks + kt - oz;
+      float w = 0.0f;
+#pragma unroll
+      for (int t = 0; t < 5; t++) w += (n1 == t ? tap_coef<KD>(t) : 0.0f) - (n2 == t ? tap_coef<KD>(t) : 0.0f);
+#pragma unroll
+      for (int cc = 0; cc < 3; cc++) sz_[cc] += w * src[top_idx(g, cc, ks, i, j)];
+    }
+  }
+  {
+    /* mac22 of plane 1 and mac24 of plane 2 */
+    const float b1 = (float)kB1, b2 = (float)kB2, b3 = (float)kB3;
+    const float w1 = KD ? (kt == 0 ? 1.0f : (kt == 1 ? -1.0f : 0.0f)) : (kt == 1 ? 1.0f : (kt == 2 ? -1.0f : 0.0f));
+    const float w2 = KD ? (kt == 0 ? b3 : (kt == 1 ? b2 : (kt == 2 ? b1 : 0.0f)))
+                        : (kt == 2 ? -b1 : (kt == 3 ? -b2 : (kt == 4 ? -b3 : 0.0f)));
+#pragma unroll
+    for (int cc = 0; cc < 3; cc++)
+      lm[cc] += w1 * src[top_idx(g, 9 + cc, 1, i, j)] + w2 * src[top_idx(g, 9 + cc, 2, i, j)];
+  }
+  float t[3][3];
+#pragma unroll
+  for (int cc = 0; cc < 3; cc++)
+#pragma unroll
+    for (int a = 0; a < 3; a++) t[cc][a] = M[0] * (M[1 + a] * sx[cc] + M[4 + a] * sy_[cc] + M[7 + a] * sz_[cc]);
+  lm[TXX] += t[0][0];
+  lm[TYY] += t[1][1];
+  lm[TZZ] += t[2][2];
+  lm[TXY] += t[0][1] + t[1][0];
+  lm[TXZ] += t[0][2] + t[2][0];
+  lm[TYZ] += t[1][2] + t[2][1];
+}
+
 /* MODE 3: A = L^T;  2: B = L^T, P = E + A;  1: A = L^T, P += B;  0: P += A + L^T.
    VC: vertical columns (xi_y, xi_z, eta_x, eta_z left out, as the forward
    box split does).
@@ -262,7 +409,7 @@ DEVI void gather_dir(float *lm, const Grid &g, const float *__restrict__ met, co
 template <int ID, int JD, int KD, int MODE, bool VC>
 __global__ void __launch_bounds__(256, 4) k_adj_stage(Grid g, const float *__restrict__ met,
                                                    const float *__restrict__ SG, const float *__restrict__ E,
-                                                   float *A, float *B, float *P, AdjPml pm) {
+                                                   float *A, float *B, float *P, AdjPml pm, const float *__restrict__ src) {
   const int i = blockIdx.x * kTileW + (int)threadIdx.x, j = blockIdx.y * 2 + (int)threadIdx.y + 3;
   const int k = (int)(blockIdx.z * 2 + threadIdx.z) + 3;
   if (i < 3 || i >= g.ni + 3 || j >= g.nj + 3 || k > g.nk2) return;
@@ -278,6 +425,7 @@ __global__ void __launch_bounds__(256, 4) k_adj_stage(Grid g, const float *__res
   __asm__ volatile("" : "+v"(lm[0]), "+v"(lm[1]), "+v"(lm[2]), "+v"(lm[3]), "+v"(lm[4]), "+v"(lm[5]),
                    "+v"(lm[6]), "+v"(lm[7]), "+v"(lm[8]) : : "memory");
   gather_dir<2, KD, -1>(lm, g, met, SG, pm, i, j, k, q);
+  if (src && g.nk2 - k <= 4) gather_top<ID, JD, KD>(lm, g, met, src, i, j, k, q);
   /* loads before stores */
   float av[9], pv[9];
 #pragma unroll
@@ -293,220 +441,6 @@ __global__ void __launch_bounds__(256, 4) k_adj_stage(Grid g, const float *__res
     else if (MODE == 2) { B[o] = lm[f]; P[o] = pv[f] + av[f]; }
     else if (MODE == 1) { A[o] = lm[f]; P[o] = pv[f] + av[f]; }
     else P[o] = pv[f] + (av[f] + lm[f]);
-  }
-}
-
-/* ------------------------------------------------------------------------
- * Adjoint of the free-surface replacements at the top four layers, added to
- * the stage's L^T output T (the level the stage kernel just wrote: A for
- * stages 3 and 1, B for stage 2, P for stage 0). One thread per point.
- * ---------------------------------------------------------------------- */
-DEVI bool phys(const Grid &g, int i, int j, int k) {
-  return i >= 3 && i < g.ni + 3 && j >= 3 && j < g.nj + 3 && k >= 3 && k <= g.nk2;
-}
-
-template <int ID, int JD, int KD, int MODE>
-__global__ void __launch_bounds__(256) k_adj_top(Grid g, const float *__restrict__ met, const float *__restrict__ lam,
-                                                 const float *__restrict__ mu, const float *__restrict__ slw,
-                                                 const float *__restrict__ mx, const float *__restrict__ my,
-                                                 const float *__restrict__ X, float alpha,
-                                                 const float *__restrict__ E, float beta, float *T, AdjPml pm) {
-  const int i = blockIdx.x * kTileW + (int)threadIdx.x, j = blockIdx.y * 4 + (int)threadIdx.y + 3;
-  const int nk2 = g.nk2;
-  const int k = nk2 - (int)blockIdx.z;  /* planes nk2, nk2-1, nk2-2, nk2-3 */
-  if (i < 3 || i >= g.ni + 3 || j >= g.nj + 3 || k < 3) return;
-  if (pm.fs.nfault > 0 && fault_column(pm.fs, i, j + (long)k * g.ny)) return;
-  const long sc = g.sicmp, sy = g.siy, sz = g.siz;
-  const long p = i + j * sy + (long)k * sz;
-  float c[9];
-#pragma unroll
-  for (int f = 0; f < 9; f++) c[f] = beta * E[f * sc + p] + (X ? alpha * X[f * sc + p] : 0.0f);
-  const float l = lam[p], m = mu[p], s = slw[p];
-  constexpr int fxo = ID ? -1 : -3, fyo = JD ? -1 : -3, fzo = KD ? -1 : -3;
-  const int tf[3][3] = {{TXX, TXY, TXZ}, {TXY, TYY, TYZ}, {TXZ, TYZ, TZZ}};
-
-  if (k >= nk2 - (fzo + 4)) {
-    /* timg: h_c = s/J(p) sum_taps coef J(q) (xi_d(q) . T_c(q)), odd image above the surface */
-    const int n_free = nk2 - k - fzo;
-    const float sj = s / met[p];
-    /* the taps' places and their coef J xi_d, for all three components at
-       once; a tap off the grid weighs zero and is placed at the point itself */
-    long dq[3][5];
-    float u[3][5][3];
-#pragma unroll
-    for (int d = 0; d < 3; d++)
-#pragma unroll
-      for (int n = 0; n < 5; n++) {
-        int off = d == 0 ? fxo + n : (d == 1 ? fyo + n : fzo + n);
-        float w = d == 0 ? tap_coef<ID>(n) : (d == 1 ? tap_coef<JD>(n) : tap_coef<KD>(n));
-        if (d == 2 && n >= n_free) {
-          if (n == n_free) w = 0.0f;  /* the surface itself */
-          off -= 2 * (n - n_free);
-          w = -w;
-        }
-        const bool in = phys(g, i + (d == 0 ? off : 0), j + (d == 1 ? off : 0), k + (d == 2 ? off : 0)) && w != 0.0f;
-        dq[d][n] = in ? off * (d == 0 ? 1 : (d == 1 ? sy : sz)) : 0;
-        const long q = p + dq[d][n];
-        const float jw = in ? w * sj * met[q] : 0.0f;
-#pragma unroll
-        for (int a = 0; a < 3; a++) u[d][n][a] = jw * met[(1 + 3 * d + a) * sc + q];
-      }
-#pragma unroll 1
-    for (int cc = 0; cc < 3; cc++) {
-      const float w = c[cc];
-      const bool bad = !(fabsf(w) < __builtin_inff());  /* not finite: also where u is zero */
-      float *T0 = T + p;
-#pragma unroll
-      for (int d = 0; d < 3; d++)
-#pragma unroll
-        for (int n = 0; n < 5; n++) {
-#pragma unroll
-          for (int a = 0; a < 3; a++)
-            if (u[d][n][a] != 0.0f || bad) atomicAdd(T0 + tf[cc][a] * sc + dq[d][n], w * u[d][n][a]);
-        }
-    }
-  }
-
-  if (k >= nk2 - 2) {
-    /* vlow: Hooke's law on dV with x/y one-sided operators and, in z, the
-       free-surface matrices (k = nk2), mac22 (nk2-1) or mac24 (nk2-2) */
-    const float l2m = (float)(l + 2.0 * m);
-    float gm[3][3];  /* adjoint of the physical gradient dV_c/dx_a */
-    gm[0][0] = l2m * c[TXX] + l * c[TYY] + l * c[TZZ];
-    gm[0][1] = m * c[TXY];
-    gm[0][2] = m * c[TXZ];
-    gm[1][0] = m * c[TXY];
-    gm[1][1] = l * c[TXX] + l2m * c[TYY] + l * c[TZZ];
-    gm[1][2] = m * c[TYZ];
-    gm[2][0] = m * c[TXZ];
-    gm[2][1] = m * c[TYZ];
-    gm[2][2] = l * c[TXX] + l * c[TYY] + l2m * c[TZZ];
-    float dl[3][3];  /* adjoint of D_d V_c */
-#pragma unroll
-    for (int d = 0; d < 3; d++)
-#pragma unroll
-      for (int cc = 0; cc < 3; cc++)
-        dl[d][cc] = met[(1 + 3 * d) * sc + p] * gm[cc][0] + met[(2 + 3 * d) * sc + p] * gm[cc][1] +
-                    met[(3 + 3 * d) * sc + p] * gm[cc][2];
-    if (k == nk2) {
-      const long ij = ((long)i + (long)j * sy) * 9;
-#pragma unroll
-      for (int cc = 0; cc < 3; cc++) {
-        float ax = 0.0f, ay = 0.0f;
-#pragma unroll
-        for (int r = 0; r < 3; r++) {
-          ax += mx[ij + 3 * r + cc] * dl[2][r];
-          ay += my[ij + 3 * r + cc] * dl[2][r];
-        }
-        dl[0][cc] += ax;
-        dl[1][cc] += ay;
-      }
-    } else {
-#pragma unroll
-      for (int cc = 0; cc < 3; cc++) {
-        float *Tc = T + cc * sc;
-        const float w = dl[2][cc];
-        if (k == nk2 - 1) {  /* mac22 */
-          if (KD) { atomicAdd(Tc + p + sz, w); atomicAdd(Tc + p, -w); }
-          else { atomicAdd(Tc + p, w); atomicAdd(Tc + p - sz, -w); }
-        } else {             /* mac24 */
-          const float b1 = (float)kB1, b2 = (float)kB2, b3 = (float)kB3;
-          if (KD) { atomicAdd(Tc + p, b1 * w); atomicAdd(Tc + p + sz, b2 * w); atomicAdd(Tc + p + 2 * sz, b3 * w); }
-          else { atomicAdd(Tc + p, -b1 * w); atomicAdd(Tc + p - sz, -b2 * w); atomicAdd(Tc + p - 2 * sz, -b3 * w); }
-        }
-      }
-    }
-#pragma unroll
-    for (int cc = 0; cc < 3; cc++)
-#pragma unroll
-      for (int t = 0; t < 5; t++) {
-        if (phys(g, i + fxo + t, j, k)) atomicAdd(T + cc * sc + p + fxo + t, tap_coef<ID>(t) * dl[0][cc]);
-        if (phys(g, i, j + fyo + t, k)) atomicAdd(T + cc * sc + p + (long)(fyo + t) * sy, tap_coef<JD>(t) * dl[1][cc]);
-      }
-  }
-
-  if (k == nk2 && pm.on) {
-    /* the free-surface term of the x/y PML faces: qT from D_dim V through
-       the matrices, added to the stress rhs with (B-1) and to the auxiliary
-       rhs with D (sv_curv_col_el_iso_gpu.cu:1000-1060, :1146-1205) */
-    const float l2m = l + 2.0f * m;
-    const float zx = met[7 * sc + p], zy = met[8 * sc + p], zz = met[9 * sc + p];
-#pragma unroll 1
-    for (int fc = 0; fc < 4; fc++) {
-      const AdjFace &F = pm.f[fc];
-      if (!in_face(F, i, j, k)) continue;
-      const long ia = face_idx(F, i, j, k), n = F.n;
-      const int ic = F.dim == 0 ? i - F.i1 : j - F.j1;
-      const float cB = F.B[ic], cD = F.D[ic];
-      const float *Ea = F.lev + (long)pm.le * 9 * n;
-      const float *Xa = MODE == 3 ? nullptr : (MODE == 1 ? F.lev + 18 * n : F.lev + 9 * n);
-      float w[9];
-#pragma unroll
-      for (int f = 3; f < 9; f++) {
-        const long o2 = f * n + ia;
-        const float ca_ = beta * Ea[o2] + (Xa ? alpha * Xa[o2] : 0.0f);
-        w[f] = (float)(cB - 1.0) * c[f] + cD * ca_;
-      }
-      /* qT -> q */
-      const float q0 = l2m * zx * w[TXX] + l * zx * w[TYY] + l * zx * w[TZZ] + m * zy * w[TXY] + m * zz * w[TXZ];
-      const float q1 = l * zy * w[TXX] + l2m * zy * w[TYY] + l * zy * w[TZZ] + m * zx * w[TXY] + m * zz * w[TYZ];
-      const float q2 = l * zz * w[TXX] + l * zz * w[TYY] + l2m * zz * w[TZZ] + m * zx * w[TXZ] + m * zy * w[TYZ];
-      const long ij = ((long)i + (long)j * sy) * 9;
-      const float *Xm = (F.dim == 0 ? mx : my) + ij;
-      float dv[3];
-#pragma unroll
-      for (int cc = 0; cc < 3; cc++) dv[cc] = Xm[cc] * q0 + Xm[3 + cc] * q1 + Xm[6 + cc] * q2;
-#pragma unroll
-      for (int cc = 0; cc < 3; cc++)
-#pragma unroll
-        for (int t = 0; t < 5; t++) {
-          if (F.dim == 0) {
-            if (phys(g, i + fxo + t, j, k)) atomicAdd(T + cc * sc + p + fxo + t, tap_coef<ID>(t) * dv[cc]);
-          } else {
-            if (phys(g, i, j + fyo + t, k)) atomicAdd(T + cc * sc + p + (long)(fyo + t) * sy, tap_coef<JD>(t) * dv[cc]);
-          }
-        }
-    }
-  }
-}
-
-template <int ID, int JD, int KD>
-static void adj_top_dir(int mode, const Grid &g, const float *met, const float *lam, const float *mu,
-                        const float *slw, const float *mx, const float *my, const float *X, float alpha,
-                        const float *E, float beta, float *T, const AdjPml &pm, hipStream_t st) {
-  dim3 blk(kTileW, 4, 1), grd(tiles_x(g), (g.nj + 3) / 4, g.nk < 4 ? g.nk : 4);
-  switch (mode) {
-    case 3:
-      hipLaunchKernelGGL((k_adj_top<ID, JD, KD, 3>), grd, blk, 0, st, g, met, lam, mu, slw, mx, my, X, alpha, E,
-                         beta, T, pm);
-      break;
-    case 2:
-      hipLaunchKernelGGL((k_adj_top<ID, JD, KD, 2>), grd, blk, 0, st, g, met, lam, mu, slw, mx, my, X, alpha, E,
-                         beta, T, pm);
-      break;
-    case 1:
-      hipLaunchKernelGGL((k_adj_top<ID, JD, KD, 1>), grd, blk, 0, st, g, met, lam, mu, slw, mx, my, X, alpha, E,
-                         beta, T, pm);
-      break;
-    default:
-      hipLaunchKernelGGL((k_adj_top<ID, JD, KD, 0>), grd, blk, 0, st, g, met, lam, mu, slw, mx, my, X, alpha, E,
-                         beta, T, pm);
-      break;
-  }
-}
-
-void launch_adj_top(int mode, int idir, int jdir, int kdir, const Grid &g, const float *met, const float *lam,
-                    const float *mu, const float *slw, const float *mx, const float *my, const float *X, float alpha,
-                    const float *E, float beta, float *T, const AdjPml &pm, hipStream_t st) {
-  switch (idir * 4 + jdir * 2 + kdir) {
-    case 0: adj_top_dir<0, 0, 0>(mode, g, met, lam, mu, slw, mx, my, X, alpha, E, beta, T, pm, st); break;
-    case 1: adj_top_dir<0, 0, 1>(mode, g, met, lam, mu, slw, mx, my, X, alpha, E, beta, T, pm, st); break;
-    case 2: adj_top_dir<0, 1, 0>(mode, g, met, lam, mu, slw, mx, my, X, alpha, E, beta, T, pm, st); break;
-    case 3: adj_top_dir<0, 1, 1>(mode, g, met, lam, mu, slw, mx, my, X, alpha, E, beta, T, pm, st); break;
-    case 4: adj_top_dir<1, 0, 0>(mode, g, met, lam, mu, slw, mx, my, X, alpha, E, beta, T, pm, st); break;
-    case 5: adj_top_dir<1, 0, 1>(mode, g, met, lam, mu, slw, mx, my, X, alpha, E, beta, T, pm, st); break;
-    case 6: adj_top_dir<1, 1, 0>(mode, g, met, lam, mu, slw, mx, my, X, alpha, E, beta, T, pm, st); break;
-    default: adj_top_dir<1, 1, 1>(mode, g, met, lam, mu, slw, mx, my, X, alpha, E, beta, T, pm, st); break;
   }
 }
 
@@ -526,56 +460,58 @@ __global__ void k_adj_inject(const long *__restrict__ term, const float *__restr
 }
 
 void launch_adj_prep(int mode, const Grid &g, const float *lam, const float *mu, const float *slw, const float *X,
-                     float alpha, const float *E, float beta, float *SG, const AdjPml &pm, int isfree, int kdir,
+                     float alpha, const float *E, float beta, float *SG, const AdjPml &pm, const AdjTop &top, int kdir,
                      hipStream_t st) {
   dim3 blk(kTileW, 4, 1), grd(tiles_x(g), (g.nj + 3) / 4, g.nk);
   switch (mode) {
     case 3:
-      hipLaunchKernelGGL(k_adj_prep<3>, grd, blk, 0, st, g, lam, mu, slw, X, alpha, E, beta, SG, pm, isfree, kdir);
+      hipLaunchKernelGGL(k_adj_prep<3>, grd, blk, 0, st, g, lam, mu, slw, X, alpha, E, beta, SG, pm, top, kdir);
       break;
     case 2:
-      hipLaunchKernelGGL(k_adj_prep<2>, grd, blk, 0, st, g, lam, mu, slw, X, alpha, E, beta, SG, pm, isfree, kdir);
+      hipLaunchKernelGGL(k_adj_prep<2>, grd, blk, 0, st, g, lam, mu, slw, X, alpha, E, beta, SG, pm, top, kdir);
       break;
     case 1:
-      hipLaunchKernelGGL(k_adj_prep<1>, grd, blk, 0, st, g, lam, mu, slw, X, alpha, E, beta, SG, pm, isfree, kdir);
+      hipLaunchKernelGGL(k_adj_prep<1>, grd, blk, 0, st, g, lam, mu, slw, X, alpha, E, beta, SG, pm, top, kdir);
       break;
     default:
-      hipLaunchKernelGGL(k_adj_prep<0>, grd, blk, 0, st, g, lam, mu, slw, X, alpha, E, beta, SG, pm, isfree, kdir);
+      hipLaunchKernelGGL(k_adj_prep<0>, grd, blk, 0, st, g, lam, mu, slw, X, alpha, E, beta, SG, pm, top, kdir);
       break;
   }
 }
 
 template <int ID, int JD, int KD, bool VC>
 static void adj_stage_dir(int mode, const Grid &g, const float *met, const float *SG, const float *E, float *A,
-                          float *B, float *P, const AdjPml &pm, hipStream_t st) {
+                          float *B, float *P, const AdjPml &pm, const float *src, hipStream_t st) {
   dim3 blk(kTileW, 2, 2), grd(tiles_x(g), (g.nj + 1) / 2, (g.nk + 1) / 2);
   switch (mode) {
-    case 3: hipLaunchKernelGGL((k_adj_stage<ID, JD, KD, 3, VC>), grd, blk, 0, st, g, met, SG, E, A, B, P, pm); break;
-    case 2: hipLaunchKernelGGL((k_adj_stage<ID, JD, KD, 2, VC>), grd, blk, 0, st, g, met, SG, E, A, B, P, pm); break;
-    case 1: hipLaunchKernelGGL((k_adj_stage<ID, JD, KD, 1, VC>), grd, blk, 0, st, g, met, SG, E, A, B, P, pm); break;
-    default: hipLaunchKernelGGL((k_adj_stage<ID, JD, KD, 0, VC>), grd, blk, 0, st, g, met, SG, E, A, B, P, pm); break;
+    case 3: hipLaunchKernelGGL((k_adj_stage<ID, JD, KD, 3, VC>), grd, blk, 0, st, g, met, SG, E, A, B, P, pm, src); break;
+    case 2: hipLaunchKernelGGL((k_adj_stage<ID, JD, KD, 2, VC>), grd, blk, 0, st, g, met, SG, E, A, B, P, pm, src); break;
+    case 1: hipLaunchKernelGGL((k_adj_stage<ID, JD, KD, 1, VC>), grd, blk, 0, st, g, met, SG, E, A, B, P, pm, src); break;
+    default: hipLaunchKernelGGL((k_adj_stage<ID, JD, KD, 0, VC>), grd, blk, 0, st, g, met, SG, E, A, B, P, pm, src); break;
   }
 }
 
 template <bool VC>
 static void adj_stage_vc(int mode, int idir, int jdir, int kdir, const Grid &g, const float *met, const float *SG,
-                         const float *E, float *A, float *B, float *P, const AdjPml &pm, hipStream_t st) {
+                         const float *E, float *A, float *B, float *P, const AdjPml &pm, const float *src,
+                         hipStream_t st) {
   switch (idir * 4 + jdir * 2 + kdir) {
-    case 0: adj_stage_dir<0, 0, 0, VC>(mode, g, met, SG, E, A, B, P, pm, st); break;
-    case 1: adj_stage_dir<0, 0, 1, VC>(mode, g, met, SG, E, A, B, P, pm, st); break;
-    case 2: adj_stage_dir<0, 1, 0, VC>(mode, g, met, SG, E, A, B, P, pm, st); break;
-    case 3: adj_stage_dir<0, 1, 1, VC>(mode, g, met, SG, E, A, B, P, pm, st); break;
-    case 4: adj_stage_dir<1, 0, 0, VC>(mode, g, met, SG, E, A, B, P, pm, st); break;
-    case 5: adj_stage_dir<1, 0, 1, VC>(mode, g, met, SG, E, A, B, P, pm, st); break;
-    case 6: adj_stage_dir<1, 1, 0, VC>(mode, g, met, SG, E, A, B, P, pm, st); break;
-    default: adj_stage_dir<1, 1, 1, VC>(mode, g, met, SG, E, A, B, P, pm, st); break;
+    case 0: adj_stage_dir<0, 0, 0, VC>(mode, g, met, SG, E, A, B, P, pm, src, st); break;
+    case 1: adj_stage_dir<0, 0, 1, VC>(mode, g, met, SG, E, A, B, P, pm, src, st); break;
+    case 2: adj_stage_dir<0, 1, 0, VC>(mode, g, met, SG, E, A, B, P, pm, src, st); break;
+    case 3: adj_stage_dir<0, 1, 1, VC>(mode, g, met, SG, E, A, B, P, pm, src, st); break;
+    case 4: adj_stage_dir<1, 0, 0, VC>(mode, g, met, SG, E, A, B, P, pm, src, st); break;
+    case 5: adj_stage_dir<1, 0, 1, VC>(mode, g, met, SG, E, A, B, P, pm, src, st); break;
+    case 6: adj_stage_dir<1, 1, 0, VC>(mode, g, met, SG, E, A, B, P, pm, src, st); break;
+    default: adj_stage_dir<1, 1, 1, VC>(mode, g, met, SG, E, A, B, P, pm, src, st); break;
   }
 }
 
 void launch_adj_stage(int mode, int idir, int jdir, int kdir, const Grid &g, const float *met, const float *SG,
-                      const float *E, float *A, float *B, float *P, const AdjPml &pm, int vcol, hipStream_t st) {
-  if (vcol) adj_stage_vc<true>(mode, idir, jdir, kdir, g, met, SG, E, A, B, P, pm, st);
-  else adj_stage_vc<false>(mode, idir, jdir, kdir, g, met, SG, E, A, B, P, pm, st);
+                      const float *E, float *A, float *B, float *P, const AdjPml &pm, const float *src, int vcol,
+                      hipStream_t st) {
+  if (vcol) adj_stage_vc<true>(mode, idir, jdir, kdir, g, met, SG, E, A, B, P, pm, src, st);
+  else adj_stage_vc<false>(mode, idir, jdir, kdir, g, met, SG, E, A, B, P, pm, src, st);
 }
 
 void launch_adj_inject(const long *term, const float *fac, int nterm, int nsta, const float *res, int nt, int n,
