@@ -25,10 +25,11 @@
  * the surface maxima at the next step start. The value the trial writes
  * onto the stage input is what the neighbours' stencils read.
  *
- * Reverse of one stage (each kernel the scatter transpose of its forward
- * gather, same lanes and addresses, atomic adds where lanes share a target):
+ * Reverse of one stage (the node kernels are the scatter transposes of their
+ * forward gathers, same lanes and addresses, with atomic adds where lanes
+ * share a target; k_adjf_cols, with by far the most taps, is a gather):
  *   k_adjf_lev   RK structure of the split-node levels (as the wavefield's)
- *   [wave prep / stage / top, fault columns left out]
+ *   [wave prep / stage, fault columns left out]
  *   k_adjf_cols  5^T into the wavefield adjoint, T1 slot 3, split velocity
  *   k_adjf_nodes 6^T into T1, neighbouring split-node state, hT1
  *   k_adjf_trial 3^T (fault2wave, friction on the taped branch, trial) and
@@ -288,178 +289,266 @@ __global__ void __launch_bounds__(kNodeLanes) k_adjf_lev(AdjFaultArgs a) {
 }
 
 /* ---------------------------------------------------------------------- */
-/* fault_cols (k_fault.hip) transposed: six lanes per node, one per column */
-constexpr int kColNodes = 10;
-
-/* The block's traction-vector adjoints (the entries the forward kernel
-   computes once into LDS: 13 x-columns, 16 y-rows and 10 z-planes around
-   its kColNodes x kColRows nodes) are accumulated in LDS by the lanes and
-   turned into stress adjoints once per entry. */
-constexpr int kColRows = 4;
-constexpr int kTvX = 13 * kColNodes * kColRows;
-constexpr int kTvY = 6 * (kColNodes + 6) * kColRows;
-constexpr int kTvZ = 6 * kColNodes * (kColRows + 6);
-constexpr int kTv = kTvX + kTvY + kTvZ;
+/* fault_cols (k_fault.hip) transposed, as a gather. A block owns the targets
+   of kColNodes x kColRows nodes (ghost rows and planes included): the twelve
+   wavefield columns the forward stencils of these rows read, and the plane.
+   Phase 1 forms, for the six column points of every node whose taps reach the
+   tile (the tile and three nodes to each side: a cross), the adjoints of the
+   traction sums and of the velocity differences; phase 2 sums each target's
+   taps from LDS and adds them to what the stage wrote, one lane to a target.
+   A scatter with atomic adds (500 to a node, and device-scope atomics leave
+   the XCD's L2) took 121 us at 240 x 100 nodes and 36.7 at 128 x 48; this
+   takes 56 and 20, with three times the loads for the cross. */
+constexpr int kColNodes = 10, kColRows = 4, kColLanes = 384;
+constexpr int kColY = (kColNodes + 6) * kColRows;            /* the tile's rows with their y halo */
+constexpr int kColSrc = kColY + kColNodes * 6;               /* and the z halo */
+DEVI void col_src(int m, int &jn, int &kr) {
+  if (m < kColY) {
+    jn = m % (kColNodes + 6) - 3;
+    kr = m / (kColNodes + 6);
+  } else {
+    jn = (m - kColY) % kColNodes;
+    kr = (m - kColY) / kColNodes;
+    kr = kr < 3 ? kr - 3 : kr - 3 + kColRows;
+  }
+}
+DEVI int col_src_z(int jn, int kr) {  /* source of tile row kr in [-3, kColRows + 3) at the tile's jn */
+  return kr >= 0 && kr < kColRows ? jn + 3 + (kColNodes + 6) * kr
+                                  : kColY + jn + kColNodes * (kr < 0 ? kr + 3 : kr + 3 - kColRows);
+}
 
 template <int IDIR>
-__global__ void __launch_bounds__(256) k_adjf_cols(AdjFaultArgs a) {
-  __shared__ float atv[3][kTv];
+__global__ void __launch_bounds__(kColLanes) k_adjf_cols(AdjFaultArgs a) {
+  __shared__ float sg[12][6 * kColSrc]; /* traction sums, D_x V, D_y V, D_z V (three components each) */
+  /* x stencils over the columns i0 - 6 .. i0 + 6 (6: the plane): cxv weights
+     D_x V; cxt[.][.][l] how often the product of tap l counts, images beyond
+     the plane included (a sum of products, not a product with a sum: far from
+     the receivers the traction sums are denormal, where products round
+     coarsely and sums are exact) */
+  __shared__ float cxt[6][13][7], cxv[6][13];
   const int id = blockIdx.z;
   const FaultDev &F = a.ftab[id];
   const long ss = a.g.sslice, sc = a.g.sicmp, sy = a.g.siy, sz = a.g.siz;
   const int i0 = F.i0;
-  const int j0 = blockIdx.x * kColNodes, k0 = blockIdx.y * kColRows;
-  const int lane = threadIdx.x, jn = lane / 6, kr = threadIdx.y;
-  const int iy = j0 + jn, iz = k0 + kr;
-  const long pf = (iy + 3) + (long)(iz + 3) * a.g.ny;
-  const bool mine = lane < 6 * kColNodes && iy < a.g.nj && iz < a.g.nk && F.united[pf] == 0;
-  if (!__syncthreads_or(mine)) return;  /* blocks of welded nodes only */
-  const int tid = threadIdx.x + 64 * threadIdx.y;
-  for (int v = tid; v < 3 * kTv; v += 64 * kColRows) (&atv[0][0])[v] = 0.0f;
-  __syncthreads();
-  const int cl = lane % 6;
-  const int mm = cl < 3 ? cl - 3 : cl - 2;
-  const int i = i0 + mm, n = -mm;
-  const long row = (long)(iy + 3) * sy + (long)(iz + 3) * sz;
-  const long p = i + row;
-  const int km = a.g.nk - (iz + 1), n_free = km + 3;
+  const int j0 = (int)blockIdx.x * kColNodes - 3, k0 = (int)blockIdx.y * kColRows - 3;
+  const int tid = threadIdx.x;
   const bool surf = a.isfree == 1;
   const float *met = a.met;
-  float *T = a.wT;
-  float *blk = adj_block(a, id);
-  float *aT1 = blk + kOffT1 * ss, *aC = adj_lev(a, blk, a.lc);
-  float hh[9];
-  if (mine) {
+  constexpr int kIt = (6 * kColSrc + kColLanes - 1) / kColLanes;
+  bool mine[kIt], any = false;
 #pragma unroll
-    for (int f = 0; f < 9; f++) hh[f] = a.cb * a.wE[f * sc + p] + (a.wX ? a.ca * a.wX[f * sc + p] : 0.0f);
-    /* velocity rhs: (dvx + dvy + dvz) slw / J over the traction vectors at
-       the taps */
-    const float rrhojac = a.slw[p] / met[p];
-#pragma unroll 1
-    for (int c = 0; c < 3; c++) {
-      const float gc = hh[c] * rrhojac;
-      float au[7];
-#pragma unroll
-      for (int l = 0; l < 7; l++) au[l] = gc * vecc_coef(l - 3, IDIR);
-      /* images beyond the plane, then the plane tap (the fault traction) */
-      if (n == 2) { au[5] += 2.0f * au[6]; au[4] -= au[6]; au[6] = 0.0f; }
-      if (n == 1) {
-        au[4] += 2.0f * au[6]; au[2] -= au[6]; au[6] = 0.0f;
-        au[4] += 2.0f * au[5]; au[3] -= au[5]; au[5] = 0.0f;
-      }
-      if (n == -1) {
-        au[2] += 2.0f * au[1]; au[3] -= au[1]; au[1] = 0.0f;
-        au[2] += 2.0f * au[0]; au[4] -= au[0]; au[0] = 0.0f;
-      }
-      if (n == -2) { au[1] += 2.0f * au[0]; au[2] -= au[0]; au[0] = 0.0f; }
-      aadd(aT1 + (long)(7 * c + 3) * ss + pf, au[n + 3]);
-      au[n + 3] = 0.0f;
-      float wz[7];
-#pragma unroll
-      for (int t = 0; t < 7; t++) wz[t] = gc * vecc_coef(t - 3, a.kdir);
-      if (surf && km <= 3) t_free_image(wz, n_free);
-#pragma unroll
-      for (int t = 0; t < 7; t++) {
-        if (au[t] != 0.0f) atomicAdd(&atv[c][mm + t + 3 + 13 * (jn + kColNodes * kr)], au[t]);
-        const float wy = gc * vecc_coef(t - 3, a.jdir);
-        if (wy != 0.0f) atomicAdd(&atv[c][kTvX + cl + 6 * (jn + t + (kColNodes + 6) * kr)], wy);
-        if (wz[t] != 0.0f) atomicAdd(&atv[c][kTvX + kTvY + cl + 6 * (jn + kColNodes * (kr + t))], wz[t]);
-      }
-    }
+  for (int it = 0; it < kIt; it++) {
+    const int v = tid + it * kColLanes;
+    int jn, kr;
+    col_src(v / 6, jn, kr);
+    const int iy = j0 + jn, iz = k0 + kr;
+    mine[it] = v < 6 * kColSrc && iy >= 0 && iy < a.g.nj && iz >= 0 && iz < a.g.nk &&
+               F.united[(iy + 3) + (long)(iz + 3) * a.g.ny] == 0;
+    any |= mine[it];
   }
-  __syncthreads();
-  /* each entry's stress adjoints: tv_c = J (a1 s_c0 + a2 s_c1 + a3 s_c2) */
-  for (int v = tid; v < kTv; v += 64 * kColRows) {
-    const float t0 = atv[0][v], t1 = atv[1][v], t2 = atv[2][v];
-    if (t0 == 0.0f && t1 == 0.0f && t2 == 0.0f) continue;
-    int x, jg, kg, d;
-    if (v < kTvX) {
-      const int xi = v % 13, r = v / 13;
-      x = i0 - 6 + xi; jg = j0 + r % kColNodes + 3; kg = k0 + r / kColNodes + 3; d = 0;
-    } else if (v < kTvX + kTvY) {
-      const int u = v - kTvX, col = u % 6, r = u / 6;
-      x = i0 + (col < 3 ? col - 3 : col - 2); jg = j0 + r % (kColNodes + 6); kg = k0 + r / (kColNodes + 6) + 3; d = 1;
-    } else {
-      const int u = v - kTvX - kTvY, col = u % 6, r = u / 6;
-      x = i0 + (col < 3 ? col - 3 : col - 2); jg = j0 + r % kColNodes + 3; kg = k0 + r / kColNodes; d = 2;
-    }
-    if (x < 0 || x >= a.g.nx || jg < 0 || jg >= a.g.ny || kg < 0 || kg >= a.g.nz) continue;
-    const long q = x + (long)jg * sy + (long)kg * sz;
-    const float jq = met[q], a1 = met[(1 + 3 * d) * sc + q], a2 = met[(2 + 3 * d) * sc + q],
-                a3 = met[(3 + 3 * d) * sc + q];
-    const float u0 = jq * t0, u1 = jq * t1, u2 = jq * t2;
-    aadd(T + TXX * sc + q, a1 * u0);
-    aadd(T + TXY * sc + q, a2 * u0 + a1 * u1);
-    aadd(T + TXZ * sc + q, a3 * u0 + a1 * u2);
-    aadd(T + TYY * sc + q, a2 * u1);
-    aadd(T + TYZ * sc + q, a3 * u1 + a2 * u2);
-    aadd(T + TZZ * sc + q, a3 * u2);
-  }
-  if (!mine) return;
+  if (!__syncthreads_or(any)) return;  /* no split node reaches the tile */
 
-  /* stress rhs: Hooke's law on the velocity differences */
-  const float l = a.lam[p], m = a.mu[p], l2m = (float)(l + 2.0 * m);
-  float aG[3][3];
-  aG[0][0] = l2m * hh[TXX] + l * hh[TYY] + l * hh[TZZ];
-  aG[1][1] = l * hh[TXX] + l2m * hh[TYY] + l * hh[TZZ];
-  aG[2][2] = l * hh[TXX] + l * hh[TYY] + l2m * hh[TZZ];
-  aG[0][1] = aG[1][0] = m * hh[TXY];
-  aG[0][2] = aG[2][0] = m * hh[TXZ];
-  aG[1][2] = aG[2][1] = m * hh[TYZ];
-  float aDx[3], aDy[3], aDz[3];
+  if (tid < 6) {
+    const int mm = tid < 3 ? tid - 3 : tid - 2, n = -mm;
+    float *cv = cxv[tid];
 #pragma unroll
-  for (int c = 0; c < 3; c++) {
-    aDx[c] = met[sc + p] * aG[c][0] + met[2 * sc + p] * aG[c][1] + met[3 * sc + p] * aG[c][2];
-    aDy[c] = met[4 * sc + p] * aG[c][0] + met[5 * sc + p] * aG[c][1] + met[6 * sc + p] * aG[c][2];
-    aDz[c] = met[7 * sc + p] * aG[c][0] + met[8 * sc + p] * aG[c][1] + met[9 * sc + p] * aG[c][2];
-  }
-  if (surf && km == 0) {
-    const long ij = ((long)i + (long)(iy + 3) * sy) * 9;
-    const float *X = a.matVx2Vz + ij, *Y = a.matVy2Vz + ij;
+    for (int x = 0; x < 13; x++) cv[x] = 0.0f;
+    for (int x = 0; x < 13; x++)
 #pragma unroll
-    for (int c = 0; c < 3; c++) {
-      aDx[c] += X[c] * aDz[0] + X[3 + c] * aDz[1] + X[6 + c] * aDz[2];
-      aDy[c] += Y[c] * aDz[0] + Y[3 + c] * aDz[1] + Y[6 + c] * aDz[2];
-    }
-  }
-#pragma unroll 1
-  for (int c = 0; c < 3; c++) {
-    float *Vc = T + c * sc;
-    t_macdrp(Vc + p, sy, a.jdir, aDy[c]);
-    if (surf && km == 0) {
-    } else if (surf && km == 1) t_mac22(Vc + p, sz, a.kdir, aDz[c]);
-    else if (surf && km == 2) t_mac24(Vc + p, sz, a.kdir, aDz[c]);
-    else t_macdrp(Vc + p, sz, a.kdir, aDz[c]);
-    const float ax = aDx[c];
-    float *Vr = Vc + row;
+      for (int l = 0; l < 7; l++) cxt[tid][x][l] = 0.0f;
+    float(*au)[7] = cxt[tid] + (mm + 3);  /* au[t]: what tap t of this column holds */
+#pragma unroll
+    for (int l = 0; l < 7; l++) au[l][l] = 1.0f;
+    /* images beyond the plane: from tap f, twice to tap g and minus once to tap h */
+    auto image = [&](int f, int g, int h) {
+#pragma unroll
+      for (int l = 0; l < 7; l++) {
+        au[g][l] += 2.0f * au[f][l];
+        au[h][l] -= au[f][l];
+        au[f][l] = 0.0f;
+      }
+    };
+    if (n == 2) image(6, 5, 4);
+    if (n == 1) { image(6, 4, 2); image(5, 4, 3); }
+    if (n == -1) { image(1, 2, 3); image(0, 2, 4); }
+    if (n == -2) image(0, 1, 2);
+    /* reduced differences towards the plane, whose split side is the tap at 6 */
     const float b1 = (float)kB1, b2 = (float)kB2, b3 = (float)kB3;
     const float c1 = (float)kC1, c2 = (float)kC2, c3 = (float)kC3, c4 = (float)kC4, c5 = (float)kC5;
+    float *q = cv + 6;
     if (IDIR == 1) {
-      if (mm == 3) t_macdrp(Vr + (i0 + 3), 1, 1, ax);
-      else if (mm == 2) t_mac24(Vr + (i0 + 2), 1, 1, ax);
-      else if (mm == 1) t_mac22(Vr + (i0 + 1), 1, 1, ax);
-      else {
-        float *vm = aC + fidx(c, 0, ss) + pf;
-        if (mm == -1) { aadd(vm, ax); aadd(Vr + (i0 - 1), -ax); }
-        else if (mm == -2) { aadd(Vr + (i0 - 2), b1 * ax); aadd(Vr + (i0 - 1), b2 * ax); aadd(vm, b3 * ax); }
-        else {
-          aadd(Vr + (i0 - 4), c1 * ax); aadd(Vr + (i0 - 3), c2 * ax); aadd(Vr + (i0 - 2), c3 * ax);
-          aadd(Vr + (i0 - 1), c4 * ax); aadd(vm, c5 * ax);
-        }
-      }
+      if (mm == -1) { q[0] = 1.0f; q[-1] = -1.0f; }
+      else if (mm == -2) { q[-2] = b1; q[-1] = b2; q[0] = b3; }
+      else if (mm == 1) { q[2] = 1.0f; q[1] = -1.0f; }
+      else if (mm == 2) { q[2] = b1; q[3] = b2; q[4] = b3; }
+      else { q[mm - 1] = c1; q[mm] = c2; q[mm + 1] = c3; q[mm + 2] = c4; q[mm + 3] = c5; }
     } else {
-      if (mm == -3) t_macdrp(Vr + (i0 - 3), 1, 0, ax);
-      else if (mm == -2) t_mac24(Vr + (i0 - 2), 1, 0, ax);
-      else if (mm == -1) t_mac22(Vr + (i0 - 1), 1, 0, ax);
-      else {
-        float *vp = aC + fidx(c, 1, ss) + pf;
-        if (mm == 1) { aadd(Vr + (i0 + 1), ax); aadd(vp, -ax); }
-        else if (mm == 2) { aadd(vp, -b3 * ax); aadd(Vr + (i0 + 1), -b2 * ax); aadd(Vr + (i0 + 2), -b1 * ax); }
-        else {
-          aadd(vp, -c5 * ax); aadd(Vr + (i0 + 1), -c4 * ax); aadd(Vr + (i0 + 2), -c3 * ax);
-          aadd(Vr + (i0 + 3), -c2 * ax); aadd(Vr + (i0 + 4), -c1 * ax);
+      if (mm == 1) { q[1] = 1.0f; q[0] = -1.0f; }
+      else if (mm == 2) { q[0] = -b3; q[1] = -b2; q[2] = -b1; }
+      else if (mm == -1) { q[-1] = 1.0f; q[-2] = -1.0f; }
+      else if (mm == -2) { q[-2] = -b1; q[-3] = -b2; q[-4] = -b3; }
+      else { q[mm + 1] = -c1; q[mm] = -c2; q[mm - 1] = -c3; q[mm - 2] = -c4; q[mm - 3] = -c5; }
+    }
+  }
+
+  /* phase 1 */
+#pragma unroll
+  for (int it = 0; it < kIt; it++) {
+    const int v = tid + it * kColLanes;
+    if (v >= 6 * kColSrc) continue;
+    float o[12];
+#pragma unroll
+    for (int e = 0; e < 12; e++) o[e] = 0.0f;
+    if (mine[it]) {
+      int jn, kr;
+      col_src(v / 6, jn, kr);
+      const int cl = v % 6, iy = j0 + jn, iz = k0 + kr;
+      const int i = i0 + (cl < 3 ? cl - 3 : cl - 2);
+      const long p = i + (long)(iy + 3) * sy + (long)(iz + 3) * sz;
+      float hh[9], mt[9];
+#pragma unroll
+      for (int f = 0; f < 9; f++) hh[f] = a.cb * a.wE[f * sc + p] + (a.wX ? a.ca * a.wX[f * sc + p] : 0.0f);
+#pragma unroll
+      for (int f = 0; f < 9; f++) mt[f] = met[(1 + f) * sc + p];
+      const float l = a.lam[p], m = a.mu[p], l2m = (float)(l + 2.0 * m);
+      /* velocity rhs: (dvx + dvy + dvz) slw / J over the traction vectors at
+         the taps */
+      const float rrhojac = a.slw[p] / met[p];
+#pragma unroll
+      for (int c = 0; c < 3; c++) o[c] = hh[c] * rrhojac;
+      /* stress rhs: Hooke's law on the velocity differences */
+      float aG[3][3];
+      aG[0][0] = l2m * hh[TXX] + l * hh[TYY] + l * hh[TZZ];
+      aG[1][1] = l * hh[TXX] + l2m * hh[TYY] + l * hh[TZZ];
+      aG[2][2] = l * hh[TXX] + l * hh[TYY] + l2m * hh[TZZ];
+      aG[0][1] = aG[1][0] = m * hh[TXY];
+      aG[0][2] = aG[2][0] = m * hh[TXZ];
+      aG[1][2] = aG[2][1] = m * hh[TYZ];
+#pragma unroll
+      for (int d = 0; d < 3; d++)
+#pragma unroll
+        for (int c = 0; c < 3; c++)
+          o[3 + 3 * d + c] = mt[3 * d] * aG[c][0] + mt[3 * d + 1] * aG[c][1] + mt[3 * d + 2] * aG[c][2];
+      if (surf && iz == a.g.nk - 1) {
+        const long ij = ((long)i + (long)(iy + 3) * sy) * 9;
+        const float *X = a.matVx2Vz + ij, *Y = a.matVy2Vz + ij;
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+          o[3 + c] += X[c] * o[9] + X[3 + c] * o[10] + X[6 + c] * o[11];
+          o[6 + c] += Y[c] * o[9] + Y[3 + c] * o[10] + Y[6 + c] * o[11];
+        }
+        o[9] = o[10] = o[11] = 0.0f;
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < 12; e++) sg[e][v] = o[e];
+  }
+  __syncthreads();
+
+  /* phase 2 */
+  float *T = a.wT;
+  float *blk = adj_block(a, id);
+  float *aT1 = blk + kOffT1 * ss, *aV = adj_lev(a, blk, a.lc) + fidx(0, IDIR == 1 ? 0 : 1, ss);
+  const bool alone = a.nfault == 1;  /* another fault's columns may be the same points */
+#pragma unroll 1
+  for (int u = tid; u < 13 * kColNodes * kColRows; u += kColLanes) {
+    const int xi = u % 13, nd = u / 13, jn = nd % kColNodes, kr = nd / kColNodes;
+    const int x = i0 - 6 + xi, jg = j0 + jn + 3, kg = k0 + kr + 3;
+    if (x < 0 || x >= a.g.nx || jg < 0 || jg >= a.g.ny || kg < 0 || kg >= a.g.nz) continue;
+    float vel[3] = {0.0f, 0.0f, 0.0f}, tx[3] = {0.0f, 0.0f, 0.0f};
+    const int m0 = 6 * (jn + 3 + (kColNodes + 6) * kr);
+#pragma unroll
+    for (int cl = 0; cl < 6; cl++) {
+      const float wv = cxv[cl][xi];
+#pragma unroll
+      for (int c = 0; c < 3; c++) {
+        const float g = sg[c][m0 + cl];
+#pragma unroll
+        for (int l = 0; l < 7; l++)
+          if (vecc_coef(l - 3, IDIR) != 0.0f) tx[c] += cxt[cl][xi][l] * __fmul_rn(g, vecc_coef(l - 3, IDIR));
+        vel[c] += wv * sg[3 + c][m0 + cl];
+      }
+    }
+    if (xi == 6) {  /* the plane: the fault traction and the split side's velocity */
+      const bool node = jg >= 3 && jg < a.g.nj + 3 && kg >= 3 && kg < a.g.nk + 3;
+      const long pf = jg + (long)kg * a.g.ny;
+      if (node && F.united[pf] == 0) {
+        float t3[3], v3[3];
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+          t3[c] = aT1[(long)(7 * c + 3) * ss + pf];
+          v3[c] = aV[2 * c * ss + pf];
+        }
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+          aT1[(long)(7 * c + 3) * ss + pf] = t3[c] + tx[c];
+          aV[2 * c * ss + pf] = v3[c] + vel[c];
         }
       }
+      continue;
+    }
+    const long q = x + (long)jg * sy + (long)kg * sz;
+    const bool near = xi >= 3 && xi <= 9;
+    float w[9], M[10];
+#pragma unroll
+    for (int f = 0; f < 9; f++) w[f] = alone ? T[f * sc + q] : 0.0f;
+#pragma unroll
+    for (int e = 0; e < 10; e++) M[e] = e < 4 || near ? met[e * sc + q] : 0.0f;
+    float ty[3] = {0.0f, 0.0f, 0.0f}, tz[3] = {0.0f, 0.0f, 0.0f};
+    if (near) {
+      const int cl = xi < 6 ? xi - 3 : xi - 4;
+#pragma unroll
+      for (int o = -3; o <= 3; o++) {
+        /* the source whose tap o this is */
+        const float wy = vecc_coef(o, a.jdir);
+        const int my = 6 * (jn - o + 3 + (kColNodes + 6) * kr) + cl;
+        const int mz = 6 * col_src_z(jn, kr - o) + cl;
+        const int km = a.g.nk - (kg - 3 - o + 1);
+        float wt = vecc_coef(o, a.kdir), wi = 0.0f, wv = wt;
+        if (surf && km <= 3) {
+          /* odd traction image about plane km above the source (t_free_image) */
+          const int im = 2 * km - o;
+          if (o >= km) wt = 0.0f;
+          else
+#pragma unroll
+            for (int t = -3; t <= 3; t++)
+              if (im == t) wi = vecc_coef(t, a.kdir);
+          /* mac22, mac24 */
+          if (km == 1) wv = a.kdir == 1 ? (o == 1 ? 1.0f : o == 0 ? -1.0f : 0.0f) : (o == 0 ? 1.0f : o == -1 ? -1.0f : 0.0f);
+          if (km == 2) {
+            const int so = a.kdir == 1 ? o : -o;
+            const float b = so == 0 ? (float)kB1 : so == 1 ? (float)kB2 : so == 2 ? (float)kB3 : 0.0f;
+            wv = a.kdir == 1 ? b : -b;
+          }
+        }
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+          ty[c] = __fadd_rn(ty[c], __fmul_rn(wy, sg[c][my]));
+          tz[c] = __fadd_rn(tz[c], __fsub_rn(__fmul_rn(wt, sg[c][mz]), __fmul_rn(wi, sg[c][mz])));
+          vel[c] += wy * sg[6 + c][my] + wv * sg[9 + c][mz];
+        }
+      }
+    }
+    /* stress adjoints of the traction vectors: tv_c = J (a1 s_c0 + a2 s_c1 + a3 s_c2);
+       J first: the sums carry 1 / J and far from the receivers are denormal */
+    float t[3][3];
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+      tx[c] *= M[0];
+      ty[c] *= M[0];
+      tz[c] *= M[0];
+#pragma unroll
+      for (int e = 0; e < 3; e++) t[c][e] = M[1 + e] * tx[c] + M[4 + e] * ty[c] + M[7 + e] * tz[c];
+    }
+    const float add[9] = {vel[0], vel[1], vel[2], t[0][0], t[1][1], t[2][2],
+                          t[1][2] + t[2][1], t[0][2] + t[2][0], t[0][1] + t[1][0]};  /* by field: V, TXX .. TXY */
+    if (alone) {
+#pragma unroll
+      for (int f = 0; f < 9; f++) T[f * sc + q] = w[f] + add[f];
+    } else {
+#pragma unroll
+      for (int f = 0; f < 9; f++)
+        if (add[f] != 0.0f) aadd(T + f * sc + q, add[f]);
     }
   }
 }
@@ -894,12 +983,13 @@ void launch_adjf_stage_pre(const AdjFaultArgs &a, hipStream_t st) {
 
 void launch_adjf_stage_post(const AdjFaultArgs &a, hipStream_t st) {
   if (a.nfault <= 0) return;
-  const dim3 cg((a.g.nj + kColNodes - 1) / kColNodes, (a.g.nk + 3) / 4, a.nfault), b(64, 4);
+  /* tiles from ghost row and plane 0 */
+  const dim3 cg((a.g.nj + 6 + kColNodes - 1) / kColNodes, (a.g.nk + 6 + kColRows - 1) / kColRows, a.nfault);
   if (a.idir == 1) {
-    hipLaunchKernelGGL(k_adjf_cols<1>, cg, b, 0, st, a);
+    hipLaunchKernelGGL(k_adjf_cols<1>, cg, dim3(kColLanes), 0, st, a);
     hipLaunchKernelGGL(k_adjf_nodes<1>, node_grid(a), dim3(kNodeLanes), 0, st, a);
   } else {
-    hipLaunchKernelGGL(k_adjf_cols<0>, cg, b, 0, st, a);
+    hipLaunchKernelGGL(k_adjf_cols<0>, cg, dim3(kColLanes), 0, st, a);
     hipLaunchKernelGGL(k_adjf_nodes<0>, node_grid(a), dim3(kNodeLanes), 0, st, a);
   }
   hipLaunchKernelGGL(k_adjf_trial, node_grid(a), dim3(kNodeLanes), 0, st, a);
