@@ -107,7 +107,7 @@ void launch_vcol_check(const Grid &g, const float *met, int *flag, hipStream_t s
 void launch_pg(const Grid &g, const BatArgs &b, const float *wend, const float *wpre, float *PG, float *Dis, float dt,
                hipStream_t st);
 
-void launch_wave2fault(const FaultArgs &a, const BatArgs &b, hipStream_t st);
+void launch_plane_in(const FaultArgs &a, const BatArgs &b, hipStream_t st);
 /* fmet[c][j + k ny] = met[c] at (i0, j, k), every ghost-inclusive (j, k) */
 void launch_fault_metric(const Grid &g, const float *met, int i0, float *fmet, hipStream_t st);
 void launch_trial(const FaultArgs &a, const BatArgs &b, hipStream_t st);

@@ -687,7 +687,7 @@ int do_step(cgfd_core *c, hipEvent_t *ev, int *nev) {
       fnew = s < 3 ? c->flev(fnewl) : nullptr;
       FaultArgs fa;
       fill_fault(c, fa, s, idir, jdir, kdir, wcur, wnew, fcur, fnew);
-      launch_wave2fault(fa, c->bat, c->st);
+      launch_plane_in(fa, c->bat, c->st);
       launch_trial(fa, c->bat, c->st);
     }
     VolArgs va;

@@ -2,8 +2,9 @@
  * k_fault.hip -- fault-plane kernels of one RK stage (one thread per fault
  * node; grid z = fault id).
  *
- *  k_wave2fault : welded nodes copy the continuum state onto both split nodes
- *                 (wave2fault_gpu, transform.cu:100-212).
+ *  k_plane_in   : welded nodes copy the continuum state onto both split nodes
+ *                 (wave2fault_gpu, transform.cu:100-212); traction vectors of
+ *                 the columns next to split nodes.
  *  k_trial      : trial traction + linear slip-weakening friction
  *                 (trial_slipweakening_gpu, trial_slipweakening.cu:91-388),
  *                 the stage accumulation of Tn/Ts1/Ts2
@@ -127,8 +128,8 @@ void launch_fault_metric(const Grid &g, const float *met, int i0, float *fmet, h
 }
 
 /* ---------------------------------------------------------------------- */
-DEVI void k_wave2fault_body(const FaultArgs &a, int id) {
-  const int iy = blockIdx.x * blockDim.x + threadIdx.x;
+DEVI void wave2fault_node(const FaultArgs &a, int id, int bx) {
+  const int iy = bx * 64 + (int)threadIdx.x;
   const int iz = blockIdx.y * blockDim.y + threadIdx.y;
   if (iy >= a.g.nj || iz >= a.g.nk) return;
   const FaultDev F = fdev(a, id);
@@ -142,6 +143,7 @@ DEVI void k_wave2fault_body(const FaultArgs &a, int id) {
   float jac = F.fmet[pf];
   float txx = W[TXX * sc + p], tyy = W[TYY * sc + p], tzz = W[TZZ * sc + p];
   float tyz = W[TYZ * sc + p], txz = W[TXZ * sc + p], txy = W[TXY * sc + p];
+  float v[3] = {W[VX * sc + p], W[VY * sc + p], W[VZ * sc + p]};
   S[0][0] = txx; S[0][1] = txy; S[0][2] = txz;
   S[1][0] = txy; S[1][1] = tyy; S[1][2] = tyz;
   S[2][0] = txz; S[2][1] = tyz; S[2][2] = tzz;
@@ -153,7 +155,6 @@ DEVI void k_wave2fault_body(const FaultArgs &a, int id) {
 #pragma unroll
   for (int c = 0; c < 3; c++) F.T1[(long)c * 7 * ss + 3 * ss + pf] = Tr[c][0];
   float *fc = a.f_cur + (long)id * 18 * ss;
-  float v[3] = {W[VX * sc + p], W[VY * sc + p], W[VZ * sc + p]};
 #pragma unroll
   for (int m = 0; m < 2; m++) {
 #pragma unroll
@@ -163,11 +164,6 @@ DEVI void k_wave2fault_body(const FaultArgs &a, int id) {
       fc[fidx(6 + c, m, ss) + pf] = Tr[c][2];
     }
   }
-}
-
-__global__ void __launch_bounds__(256) k_wave2fault(FaultArgs a, BatArgs b) {
-  const int id = (int)blockIdx.z % a.nfault;
-  k_wave2fault_body(fault_at(a, b, b.act[blockIdx.z / a.nfault]), id);
 }
 
 /* split-node average back onto the wavefield column i0 (transform.cu:331-372),
@@ -213,10 +209,10 @@ DEVI void fault2wave_node(const FaultArgs &a, const float *fm, const float *t1, 
    nodes per wavefront, so a node's loads are adjacent addresses. */
 constexpr int kTrialNodes = 10;
 
-DEVI void k_trial_t1_body(const FaultArgs &a, int id) {
+DEVI void trial_t1_node(const FaultArgs &a, int id, int bx) {
   const int lane = threadIdx.x;
   if (lane >= 6 * kTrialNodes) return;
-  const int iy = blockIdx.x * kTrialNodes + lane / 6;
+  const int iy = bx * kTrialNodes + lane / 6;
   const int cl = lane % 6;
   const int iz = blockIdx.y * blockDim.y + threadIdx.y;
   if (iy >= a.g.nj || iz >= a.g.nk) return;
@@ -245,9 +241,15 @@ DEVI void k_trial_t1_body(const FaultArgs &a, int id) {
   F.T1[14 * ss + slot * ss + pf] = jl * (x1 * txz + x2 * tyz + x3 * tzz);
 }
 
-__global__ void __launch_bounds__(256) k_trial_t1(FaultArgs a, BatArgs b) {
-  const int id = (int)blockIdx.z % a.nfault;
-  k_trial_t1_body(fault_at(a, b, b.act[blockIdx.z / a.nfault]), id);
+/* what a stage takes from its input level: block columns [0, nt1) the traction
+   columns of split nodes, the rest wave2fault at welded nodes. They touch
+   different nodes, and each alone is little more than a launch (at 120 x 60
+   nodes 9.1 + 5.1 us, together 9.2). */
+__global__ void __launch_bounds__(256) k_plane_in(FaultArgs a, BatArgs b, int nt1) {
+  const int id = (int)blockIdx.z % a.nfault, bx = (int)blockIdx.x;
+  const FaultArgs f = fault_at(a, b, b.act[blockIdx.z / a.nfault]);
+  if (bx < nt1) trial_t1_node(f, id, bx);
+  else wave2fault_node(f, id, bx - nt1);
 }
 
 /* ---------------------------------------------------------------------- */
@@ -277,7 +279,7 @@ DEVI void k_trial_body(const FaultArgs &a, int id) {
     float jac0 = fm[0];
     float rho = F.rho_f[m * ss + pf];
     Mrho[m] = (float)(0.5 * jac0 * rho);
-    float t1[3][3];  /* [comp][l-1]: the traction columns k_trial_t1 wrote */
+    float t1[3][3];  /* [comp][l-1]: the traction columns k_plane_in wrote */
 #pragma unroll
     for (int l = 1; l <= 3; l++) {
       const long slot = 3 + (2 * m - 1) * l;
@@ -981,15 +983,14 @@ __global__ void k_record(BatArgs b, const float *w, long sicmp, const long *term
 }
 
 /* ---------------------------------------------------------------------- */
-void launch_wave2fault(const FaultArgs &a, const BatArgs &b, hipStream_t st) {
+void launch_plane_in(const FaultArgs &a, const BatArgs &b, hipStream_t st) {
   if (a.nfault <= 0) return;
-  dim3 blk(64, 4, 1), grd((a.g.nj + 63) / 64, (a.g.nk + 3) / 4, a.nfault * b.nact);
-  hipLaunchKernelGGL(k_wave2fault, grd, blk, 0, st, a, b);
+  const int nt1 = (a.g.nj + kTrialNodes - 1) / kTrialNodes;
+  const dim3 grd(nt1 + (a.g.nj + 63) / 64, (a.g.nk + 3) / 4, a.nfault * b.nact);
+  hipLaunchKernelGGL(k_plane_in, grd, dim3(64, 4, 1), 0, st, a, b, nt1);
 }
 void launch_trial(const FaultArgs &a, const BatArgs &b, hipStream_t st) {
   if (a.nfault <= 0) return;
-  dim3 tblk(64, 4, 1), tgrd((a.g.nj + kTrialNodes - 1) / kTrialNodes, (a.g.nk + 3) / 4, a.nfault * b.nact);
-  hipLaunchKernelGGL(k_trial_t1, tgrd, tblk, 0, st, a, b);
   dim3 blk(64, 1, 1), grd((a.g.nj + 63) / 64, a.g.nk, a.nfault * b.nact);
   switch (a.jdir * 2 + a.kdir) {
     case 0: hipLaunchKernelGGL((k_trial<0, 0>), grd, blk, 0, st, a, b); break;
