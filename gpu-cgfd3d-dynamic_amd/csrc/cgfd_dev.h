@@ -236,6 +236,9 @@ DEVI float norm3(const float *A) {
   float x2 = A[0] * A[0], y2 = A[1] * A[1], z2 = A[2] * A[2];
   return sqrtf(x2 + y2 + z2);
 }
+/* a gathered tap; one that weighs nothing passes on no NaN or infinity */
+DEVI float tap_mul(float w, float x) { return w != 0.0f ? w * x : 0.0f; }
+
 DEVI void inv3(float m[3][3]) {
   double v[3][3];
   v[0][0] = (float)(m[1][1] * m[2][2] - m[2][1] * m[1][2]);

@@ -156,10 +156,10 @@ struct cgfd_core {
     gexec = nullptr;
   }
 
-  /* discrete adjoint: 4 levels of 9 fields (E, A, B, P) and the 12 fields
-     of the adjoint gradient terms; allocated by the first backward call */
+  /* discrete adjoint: 4 levels of 9 fields (E, A, B, P) and the 9 fields of
+     the adjoint gradient terms (with the top-layer sums behind them); allocated by the first backward call */
   float *adj = nullptr, *adj_sg = nullptr;
-  float *adj_pml = nullptr;  /* per CFS-PML face: 4 adjoint levels [9][n] + extra S, G [12][n] */
+  float *adj_pml = nullptr;  /* per CFS-PML face: 4 adjoint levels [9][n] + extra S, G [9][n] */
   /* fault part of the adjoint: the friction tape written by the forward
      kernels over the recorded window, and per fault the adjoint blocks of
      kAdjFaultFloats per node (fault state levels E, A, B, P; T1; hT1; mT1;

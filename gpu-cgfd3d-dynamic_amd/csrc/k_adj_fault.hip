@@ -466,7 +466,7 @@ __global__ void __launch_bounds__(kColLanes) k_adjf_cols(AdjFaultArgs a) {
 #pragma unroll
         for (int l = 0; l < 7; l++)
           if (vecc_coef(l - 3, IDIR) != 0.0f) tx[c] += cxt[cl][xi][l] * __fmul_rn(g, vecc_coef(l - 3, IDIR));
-        vel[c] += wv * sg[3 + c][m0 + cl];
+        vel[c] += tap_mul(wv, sg[3 + c][m0 + cl]);
       }
     }
     if (xi == 6) {  /* the plane: the fault traction and the split side's velocity */
@@ -525,7 +525,7 @@ __global__ void __launch_bounds__(kColLanes) k_adjf_cols(AdjFaultArgs a) {
         for (int c = 0; c < 3; c++) {
           ty[c] = __fadd_rn(ty[c], __fmul_rn(wy, sg[c][my]));
           tz[c] = __fadd_rn(tz[c], __fsub_rn(__fmul_rn(wt, sg[c][mz]), __fmul_rn(wi, sg[c][mz])));
-          vel[c] += wy * sg[6 + c][my] + wv * sg[9 + c][mz];
+          vel[c] += tap_mul(wy, sg[6 + c][my]) + tap_mul(wv, sg[9 + c][mz]);
         }
       }
     }

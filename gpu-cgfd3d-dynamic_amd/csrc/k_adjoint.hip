@@ -374,7 +374,7 @@ DEVI void gather_top(float *lm, const Grid &g, const float *__restrict__ met, co
 #pragma unroll
       for (int t = 0; t < 5; t++) w += (n1 == t ? tap_coef<KD>(t) : 0.0f) - (n2 == t ? tap_coef<KD>(t) : 0.0f);
 #pragma unroll
-      for (int cc = 0; cc < 3; cc++) sz_[cc] += w * src[top_idx(g, cc, ks, i, j)];
+      for (int cc = 0; cc < 3; cc++) sz_[cc] += tap_mul(w, src[top_idx(g, cc, ks, i, j)]);
     }
   }
   {
@@ -385,7 +385,7 @@ DEVI void gather_top(float *lm, const Grid &g, const float *__restrict__ met, co
                         : (kt == 2 ? -b1 : (kt == 3 ? -b2 : (kt == 4 ? -b3 : 0.0f)));
 #pragma unroll
     for (int cc = 0; cc < 3; cc++)
-      lm[cc] += w1 * src[top_idx(g, 9 + cc, 1, i, j)] + w2 * src[top_idx(g, 9 + cc, 2, i, j)];
+      lm[cc] += tap_mul(w1, src[top_idx(g, 9 + cc, 1, i, j)]) + tap_mul(w2, src[top_idx(g, 9 + cc, 2, i, j)]);
   }
   float t[3][3];
 #pragma unroll

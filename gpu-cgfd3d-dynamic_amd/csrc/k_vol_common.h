@@ -215,22 +215,6 @@ DEVI void rk_point32(const VolArgs &a, unsigned o, const float *h, long woff = 0
   rk_part32<6, 3>(a, o, h + 6, woff);
 }
 
-/* rhs + PML + RK update of one point from its 27 derivatives */
-DEVI void vol_point_update(const VolArgs &a, int i, int j, int k, long p, const float *Dx, const float *Dy,
-                           const float *Dz) {
-  const long sc = a.g.sicmp;
-  const float *M = a.met;
-  float xx = M[sc + p], xy = M[2 * sc + p], xz = M[3 * sc + p];
-  float ex = M[4 * sc + p], ey = M[5 * sc + p], ez = M[6 * sc + p];
-  float zx = M[7 * sc + p], zy = M[8 * sc + p], zz = M[9 * sc + p];
-  float l = a.lam[p], m = a.mu[p], s = a.slw[p];
-  float h[9];
-  rhs_interior(Dx, Dy, Dz, xx, xy, xz, ex, ey, ez, zx, zy, zz, l, m, s, h);
-  if (a.pml_on) pml_point(a, i, j, k, p, Dx, Dy, Dz, l, m, s, h);
-  if (a.fs.nfault > 0 && fault_column(a.fs, i, j + (long)k * a.g.ny)) return;
-  rk_point(a, p, h);
-}
-
 }  // namespace cgfd
 
 #endif
