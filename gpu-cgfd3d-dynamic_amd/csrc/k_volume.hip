@@ -972,11 +972,12 @@ static void launch_box_split(int tw, bool sweeps, bool grouped, bool one, const 
   if (one) {
     box_split(a, 64, false, x, r);
     const int w = x.x1 - x.x0;
-    const bool plane = (long)w * (x.y1 - x.y0) <= kOneLaunchPlane && st == st_pml && (VC || !grouped);
+    const bool plane = (long)w * (x.y1 - x.y0) <= kOneLaunchPlane && (VC || !grouped);
+    const bool alone = plane && st == st_pml;
     /* 32-wide tiles where 64-wide ones would idle more than a tenth of their
        lanes (a box of 224 columns, 300 x 500 x 80: 3% off the step) */
-    if (10 * w < 9 * 64 * x.ntx && (plane || b.nact == 1)) tw = 32;
-    if (plane) {
+    if (10 * w < 9 * 64 * x.ntx && (alone || b.nact == 1)) tw = 32;
+    if (alone) {
       if (tw == 32) box_split(a, 32, false, x, r);
       const unsigned per = (unsigned)((long)x.ntx * x.nty * (x.k1 - x.k0) + r[0].cum[r[0].n]);
       const dim3 grd(per * (unsigned)b.nact);
@@ -986,6 +987,9 @@ static void launch_box_split(int tw, bool sweeps, bool grouped, bool one, const 
         hipLaunchKernelGGL((k_vol_split<ID, JD, KD, 32, VC>), grd, dim3(256), 0, st, a, b, x, r[0], per);
       return;
     }
+    /* under the stage fork the box and the bands are on two streams: two
+       launches of the same sums, since the fork may not change the rounding */
+    if (plane) grouped = false;
   }
   box_split(a, tw, grouped, x, r);
   if (b.nact > 1 && sweeps && x.ntx > 0) {  /* variant 32: per-scenario slab sweeps of the box (64 x 4 tiles) */

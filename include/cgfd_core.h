@@ -341,8 +341,8 @@ int cgfd_core_run_timed(cgfd_core *core, int nsteps, float *ms_total,
    directions their points can lie in; 32 = 23 on one scenario; 33 = 23
    with every band in one launch that handles all three directions, and,
    where a plane of the box has at most 48000 points, the box in that launch
-   too (a batch on 32 or 33 as well, on vertical columns; not under the stage
-   fork); 33 takes 32-wide tiles where 64-wide ones would idle over a tenth
+   too (a batch on 32 or 33 as well, on vertical columns; under the stage
+   fork the same sums in two launches); 33 takes 32-wide tiles where 64-wide ones would idle over a tenth
    of their lanes. Batches with more than one active
    scenario run, for 20, the interior tiles with the scenarios back to back
    (XCD-contiguous) and the PML tiles in one slab-ordered sweep per
