@@ -653,9 +653,11 @@ void fill_fault(cgfd_core *c, FaultArgs &f, int istage, int idir, int jdir, int 
 
 /* volume kernel variants (see cgfd_core_set_variant): 1 direct loads; 20
    an interior kernel in slab order and a lean kernel for the tiles touching
-   a CFS-PML slab; 23, 24, 32 and 33 the box split */
+   a CFS-PML slab; 23, 24, 32 and 33 the box split (32, a batch's, is 23 on
+   a core of one scenario) */
 void launch_vol(cgfd_core *c, const VolArgs &va, int idir, int jdir, int kdir) {
-  launch_volume(c->variant, va, c->bat, idir, jdir, kdir, 0, c->st, c->st_pml());
+  const int variant = c->variant == 32 && c->nscen == 1 ? 23 : c->variant;
+  launch_volume(variant, va, c->bat, idir, jdir, kdir, 0, c->st, c->st_pml());
 }
 
 /* one time step; if ev != nullptr, event pairs bracket the volume launches */
@@ -1662,7 +1664,7 @@ extern "C" int cgfd_core_autotune(cgfd_core *c, int reps, int *variant_out, int 
   HIPCHK(hipEventCreate(&e0));
   HIPCHK(hipEventCreate(&e1));
   /* 32 differs from 23 on batches only */
-  const std::vector<int> variants = c->bat.nact > 1 ? std::vector<int>{23, 32, 33, 24, 20, 1} : std::vector<int>{23, 33, 24, 20, 1};
+  const std::vector<int> variants = c->nscen > 1 ? std::vector<int>{23, 32, 33, 24, 20, 1} : std::vector<int>{23, 33, 24, 20, 1};
   const int chunks[4] = {4, 8, 16, 32};
   float best = 1e30f;
   int bv = c->variant, bz = c->zchunk;

@@ -338,12 +338,14 @@ int cgfd_core_run_timed(cgfd_core *core, int nsteps, float *ms_total,
    bounds on 32-column boundaries; 64 x 4 tiles for 23, 32 x 8 for 24; slab
    order) and the lean PML kernel over the up to six slabs around them in
    32 x 8 tiles, launched in up to four groups by the CFS-PML face
-   directions their points can lie in; 32 = 23 on one scenario; 33 = 23
-   with every band in one launch that handles all three directions, and,
-   where a plane of the box has at most 48000 points, the box in that launch
-   too (a batch on 32 or 33 as well, on vertical columns; under the stage
-   fork the same sums in two launches); 33 takes 32-wide tiles where 64-wide ones would idle over a tenth
-   of their lanes. Batches with more than one active
+   directions their points can lie in; 32 = 23 on a core of one scenario;
+   33 = 23 with every band in one launch that handles all three directions,
+   and, where a plane of the box has at most 48000 points, the box in that
+   launch too (under the stage fork the same sums in two launches); 33 takes
+   32-wide tiles where 64-wide ones would idle over a tenth of their lanes.
+   A batch on 33, and on vertical columns one on 32, takes this one-launch
+   form as well, however many of its scenarios are active. Otherwise batches
+   with more than one active
    scenario run, for 20, the interior tiles with the scenarios back to back
    (XCD-contiguous) and the PML tiles in one slab-ordered sweep per
    scenario; for 23, 24 and 33 the box split the same way (interior tiles with
