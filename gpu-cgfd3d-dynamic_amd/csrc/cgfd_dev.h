@@ -238,6 +238,8 @@ DEVI float norm3(const float *A) {
 }
 /* a gathered tap; one that weighs nothing passes on no NaN or infinity */
 DEVI float tap_mul(float w, float x) { return w != 0.0f ? w * x : 0.0f; }
+/* the same as a factor, where the product must round as it does without */
+DEVI float tap_val(float w, float x) { return w != 0.0f ? x : 0.0f; }
 
 DEVI void inv3(float m[3][3]) {
   double v[3][3];

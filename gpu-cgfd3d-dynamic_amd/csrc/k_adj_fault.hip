@@ -90,7 +90,7 @@ DEVI void t_free_image(float *v, int n_free) {
 DEVI void t_dz_free_image(float *col, long ny, int n_free, int kdir, float a) {
   float v[7];
 #pragma unroll
-  for (int l = 0; l < 7; l++) v[l] = a * vecc_coef(l - 3, kdir);
+  for (int l = 0; l < 7; l++) v[l] = tap_val(vecc_coef(l - 3, kdir), a) * vecc_coef(l - 3, kdir);
   t_free_image(v, n_free);
 #pragma unroll
   for (int l = 0; l < 7; l++)
@@ -465,7 +465,10 @@ __global__ void __launch_bounds__(kColLanes) k_adjf_cols(AdjFaultArgs a) {
         const float g = sg[c][m0 + cl];
 #pragma unroll
         for (int l = 0; l < 7; l++)
-          if (vecc_coef(l - 3, IDIR) != 0.0f) tx[c] += cxt[cl][xi][l] * __fmul_rn(g, vecc_coef(l - 3, IDIR));
+          if (vecc_coef(l - 3, IDIR) != 0.0f) {
+            const float w = cxt[cl][xi][l];
+            tx[c] += w * tap_val(w, __fmul_rn(g, vecc_coef(l - 3, IDIR)));
+          }
         vel[c] += tap_mul(wv, sg[3 + c][m0 + cl]);
       }
     }
@@ -523,8 +526,9 @@ __global__ void __launch_bounds__(kColLanes) k_adjf_cols(AdjFaultArgs a) {
         }
 #pragma unroll
         for (int c = 0; c < 3; c++) {
-          ty[c] = __fadd_rn(ty[c], __fmul_rn(wy, sg[c][my]));
-          tz[c] = __fadd_rn(tz[c], __fsub_rn(__fmul_rn(wt, sg[c][mz]), __fmul_rn(wi, sg[c][mz])));
+          const float gy = sg[c][my], gz = sg[c][mz];
+          ty[c] = __fadd_rn(ty[c], __fmul_rn(wy, tap_val(wy, gy)));
+          tz[c] = __fadd_rn(tz[c], __fsub_rn(__fmul_rn(wt, tap_val(wt, gz)), __fmul_rn(wi, tap_val(wi, gz))));
           vel[c] += tap_mul(wy, sg[6 + c][my]) + tap_mul(wv, sg[9 + c][mz]);
         }
       }
