@@ -98,6 +98,10 @@ DEVI FaultDev fdev(const FaultArgs &a, int id) {
    blocks on st_pml (nullptr = st); the two write disjoint points */
 void launch_volume(int variant, const VolArgs &a, const BatArgs &b, int idir, int jdir, int kdir, int top,
                    hipStream_t st, hipStream_t st_pml = nullptr);
+/* does the variant run the interior box and the CFS-PML bands of a's planes
+   as one launch (without slabs, so without regard to a.zchunk); fork: with
+   st_pml a stream of its own */
+bool volume_one_launch(int variant, const VolArgs &a, int fork);
 void launch_dvh2dvz(const Grid &g, const float *met, const float *lam, const float *mu, float *mx, float *my,
                     hipStream_t st);
 /* *flag (device, zeroed by the caller) becomes nonzero if at some physical

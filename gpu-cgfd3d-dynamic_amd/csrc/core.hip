@@ -17,6 +17,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <algorithm>
+#include <array>
 #include <cstring>
 #include <map>
 #include <mutex>
@@ -48,6 +49,8 @@ const float kRkA[3] = {0.5f, 0.5f, 1.0f};
 const float kRkB[4] = {(float)(1.0 / 6.0), (float)(1.0 / 3.0), (float)(1.0 / 3.0), (float)(1.0 / 6.0)};
 const int kPairs[8][3] = {{0, 0, 0}, {1, 1, 0}, {1, 1, 1}, {0, 0, 1}, {0, 1, 0}, {1, 0, 0}, {1, 0, 1}, {0, 1, 1}};
 
+constexpr int kZchunk = 8;  /* y-tiles per slab of a schedule that was not tuned */
+
 struct DevBuf {
   std::vector<void *> ptrs;
   ~DevBuf() {
@@ -67,7 +70,7 @@ struct cgfd_core {
   int vcol_grid = 0;  /* xi_y, xi_z, eta_x, eta_z below 2^-32 of xi_x, eta_y everywhere */
   int vcol_on = 1;    /* use the vertical-column form where the grid has it */
   int variant = 33;
-  int zchunk = 4;
+  int zchunk = kZchunk;
   int nvol = 0;
   DevBuf mem;
 
@@ -1544,28 +1547,46 @@ extern "C" int cgfd_batch_active(cgfd_core *c) {
 
 /* ---- autotuned schedules, per problem shape ---- */
 namespace {
+/* what a schedule's speed depends on: the shape, and what the box split's
+   dispatch reads besides: the metric form in use, the stage fork and the
+   CFS-PML layers (which bound the box). An entry without those three (form =
+   -1) serves every core of its shape that has no entry of its own. */
 struct TuneKey {
   int ni, nj, nk, nscen, nfault, isfree, pml;
-  bool operator<(const TuneKey &o) const {
-    const int a[7] = {ni, nj, nk, nscen, nfault, isfree, pml}, b[7] = {o.ni, o.nj, o.nk, o.nscen, o.nfault, o.isfree, o.pml};
-    return std::lexicographical_compare(a, a + 7, b, b + 7);
+  int form = -1, layers[6] = {};  /* form: 1 vertical columns in use, + 2 under the stage fork */
+  std::array<int, 14> all() const {
+    return {ni, nj, nk, nscen, nfault, isfree, pml, form, layers[0], layers[1], layers[2], layers[3], layers[4], layers[5]};
   }
+  bool operator<(const TuneKey &o) const { return all() < o.all(); }
 };
-std::map<TuneKey, std::pair<int, int>> g_tuned;  /* shape -> (variant, zchunk) */
+std::map<TuneKey, std::pair<int, int>> g_tuned;  /* problem -> (variant, zchunk) */
 bool g_tune_file_read = false;
 std::mutex g_tune_mu;
 
-TuneKey tune_key(const cgfd_core *c) {
+/* the problem without metric form, fork and layers */
+TuneKey tune_shape(const cgfd_core *c) {
   int pml = 0;
   for (int d = 0; d < 3; d++)
     for (int e = 0; e < 2; e++) pml |= (c->pml[d][e].on ? 1 : 0) << (2 * d + e);
   return TuneKey{c->g.ni, c->g.nj, c->g.nk, c->nscen, c->nfault, c->isfree, pml};
 }
 
+TuneKey tune_key(const cgfd_core *c) {
+  TuneKey k = tune_shape(c);
+  k.form = (c->vcol_grid && c->vcol_on ? 1 : 0) + (c->overlap ? 2 : 0);
+  for (int d = 0; d < 3; d++)
+    for (int e = 0; e < 2; e++) {
+      const PmlFace &f = c->pml[d][e];
+      if (f.on) k.layers[2 * d + e] = d == 0 ? f.i2 - f.i1 + 1 : (d == 1 ? f.j2 - f.j1 + 1 : f.k2 - f.k1 + 1);
+    }
+  return k;
+}
+
 bool valid_variant(int v) { return v == 1 || v == 20 || v == 23 || v == 24 || v == 32 || v == 33; }
 
-/* the cache file: one "ni nj nk nscen nfault isfree pml variant zchunk" line
-   per tuned shape; later lines win */
+/* the cache file: one "ni nj nk nscen nfault isfree pml form l0 .. l5 variant
+   zchunk" line per tuned problem, l0 .. l5 the layers of the x, y and z faces,
+   or, as older files have it, one without form and layers; later lines win */
 void read_tune_file() {
   if (g_tune_file_read) return;
   g_tune_file_read = true;
@@ -1573,11 +1594,23 @@ void read_tune_file() {
   if (!path || !*path) return;
   FILE *f = std::fopen(path, "r");
   if (!f) return;
-  TuneKey k;
-  int v, z;
-  while (std::fscanf(f, "%d %d %d %d %d %d %d %d %d", &k.ni, &k.nj, &k.nk, &k.nscen, &k.nfault, &k.isfree, &k.pml,
-                     &v, &z) == 9)
+  char line[512];
+  while (std::fgets(line, sizeof line, f)) {
+    int q[17], n = 0;
+    for (char *s = line, *e; n < 17; s = e, n++) {
+      const long v = std::strtol(s, &e, 10);
+      if (e == s) break;
+      q[n] = (int)v;
+    }
+    if (n != 9 && n != 16) continue;
+    TuneKey k{q[0], q[1], q[2], q[3], q[4], q[5], q[6]};
+    if (n == 16) {
+      k.form = q[7];
+      std::copy(q + 8, q + 14, k.layers);
+    }
+    const int v = q[n - 2], z = q[n - 1];
     if (valid_variant(v) && z >= 4 && z <= 4096) g_tuned[k] = {v, z};
+  }
   std::fclose(f);
 }
 
@@ -1587,24 +1620,26 @@ void record_tuned(const TuneKey &k, int v, int z) {
   if (!path || !*path) return;
   FILE *f = std::fopen(path, "a");
   if (!f) return;
-  std::fprintf(f, "%d %d %d %d %d %d %d %d %d\n", k.ni, k.nj, k.nk, k.nscen, k.nfault, k.isfree, k.pml, v, z);
+  for (int q : k.all()) std::fprintf(f, "%d ", q);
+  std::fprintf(f, "%d %d\n", v, z);
   std::fclose(f);
 }
 }  // namespace
 
-/* variant 0: the tuned choice for this shape, else the box split with 8
+/* variant 0: the tuned choice for this problem, else the box split with 8
    y-tiles per slab: 33 (the bands in one launch) on one scenario, 32 (the
    interior box, too, in per-scenario sweeps) on a batch */
 static void apply_auto_variant(cgfd_core *c) {
   std::lock_guard<std::mutex> lk(g_tune_mu);
   read_tune_file();
   auto it = g_tuned.find(tune_key(c));
+  if (it == g_tuned.end()) it = g_tuned.find(tune_shape(c));
   if (it != g_tuned.end()) {
     c->variant = it->second.first;
     c->zchunk = it->second.second;
   } else {
     c->variant = c->nscen > 1 ? 32 : 33;
-    c->zchunk = 8;
+    c->zchunk = kZchunk;
   }
 }
 
@@ -1685,6 +1720,11 @@ extern "C" int cgfd_core_autotune(cgfd_core *c, int reps, int *variant_out, int 
         va[s].k_lo = 0;
         va[s].nk_run = c->nvol;
       }
+      /* box and bands in one launch: the z-chunk has no effect, and on a
+         batch 33 is what 32 is */
+      if (volume_one_launch(v, va[0], c->overlap) &&
+          (z != kZchunk || (v == 33 && c->nscen > 1 && volume_one_launch(32, va[0], c->overlap))))
+        continue;
       auto one = [&]() {
         for (int s = 0; s < 4; s++) {
           (void)c->fork();

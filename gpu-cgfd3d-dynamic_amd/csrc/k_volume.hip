@@ -624,6 +624,20 @@ static void box_split(const VolArgs &a, int tw, bool grouped, VolBox &x, VolBand
   add(3, xl, xr, yl, yr, kr, kv1);
 }
 
+/* is a plane of the box small enough for the one-launch form (variants 32,
+   whose bands are grouped, and 33) */
+static bool one_launch_plane(bool vcol, bool grouped, const VolBox &x) {
+  return (long)(x.x1 - x.x0) * (x.y1 - x.y0) <= kOneLaunchPlane && (vcol || !grouped);
+}
+
+bool volume_one_launch(int variant, const VolArgs &a, int fork) {
+  if ((variant != 32 && variant != 33) || fork) return false;
+  VolBox x;
+  VolBands r[kBandGroups];
+  box_split(a, 64, false, x, r);
+  return one_launch_plane(a.vcol, variant == 32, x);
+}
+
 /* The box split in one launch (variants 32 and 33 where a plane of the
    interior box is small): block ids [0, nband) of a scenario's per are the
    bands (the longer blocks first), the rest the box in TW x 256/TW tiles, x
@@ -972,7 +986,7 @@ static void launch_box_split(int tw, bool sweeps, bool grouped, bool one, const 
   if (one) {
     box_split(a, 64, false, x, r);
     const int w = x.x1 - x.x0;
-    const bool plane = (long)w * (x.y1 - x.y0) <= kOneLaunchPlane && (VC || !grouped);
+    const bool plane = one_launch_plane(VC, grouped, x);
     const bool alone = plane && st == st_pml;
     /* 32-wide tiles where 64-wide ones would idle more than a tenth of their
        lanes (a box of 224 columns, 300 x 500 x 80: 3% off the step) */

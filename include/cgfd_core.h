@@ -383,12 +383,17 @@ int cgfd_core_set_vertical_columns(cgfd_core *core, int on);
 int cgfd_core_get_vertical_columns(const cgfd_core *core, int *grid, int *in_use);
 
 /* Autotuner: times every candidate (variant, z-chunk) pair -- 23, 33, 24,
-   20 and 1, and 32 on a batch, z-chunks 4..32 for the slab-ordered ones -- on
+   20 and 1, and 32 on a batch, z-chunks 4..32 for the slab-ordered ones (8
+   where box and bands are one launch, which has no slabs) -- on
    `reps` repetitions
    of one step's four volume launches, keeps
-   the fastest and records it for this problem shape (grid, scenarios,
-   faults, boundaries) so later cores of the same shape start with it, and
-   appends it to the file named by CGFD_TUNE_CACHE if that is set; *ms_best
+   the fastest and records it for this problem (grid, scenarios, faults,
+   boundaries with their CFS-PML layers, metric form in use, stage fork) so
+   later cores of the same problem start with it (a core's fork is off when
+   it is created: after cgfd_core_set_overlap, variant 0 takes what was
+   recorded with it), and appends it to the file named by CGFD_TUNE_CACHE if
+   that is set; an older file's lines, without layers, form and fork, serve
+   every core of their shape that has no line of its own; *ms_best
    is the average per launch. The launches read level "pre" and write only
    levels that the next step rewrites before reading, so the simulation
    state is unchanged. */
