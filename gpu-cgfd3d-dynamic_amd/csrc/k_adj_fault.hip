@@ -86,7 +86,7 @@ DEVI void t_free_image(float *v, int n_free) {
   }
   v[n_free] = 0.0f;
 }
-/* dz_free_image (k_fault.hip) transposed onto the column at col */
+/* the free-surface image t_free (k_fault.hip) transposed onto the column at col */
 DEVI void t_dz_free_image(float *col, long ny, int n_free, int kdir, float a) {
   float v[7];
 #pragma unroll

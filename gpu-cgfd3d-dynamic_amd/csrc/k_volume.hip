@@ -542,12 +542,25 @@ __global__ void __launch_bounds__(256, 5) k_vol_bat_pml_band(VolArgs a, BatArgs 
 
 /* Largest plane of the interior box (points) for the one-launch form, which
    runs the box plane by plane and at the bands' 5 waves per SIMD instead of
-   8. A batch takes it on vertical columns alone; with nine metric terms its
-   bands stay in the groups of variant 32, whose sums round differently.
-   Against the two kernels: 0.674 against 0.693 ms per stage at 200 x 400 x
-   150 (a plane of 45800 points); at 260 x 400 x 80 (68700, nine metric terms)
-   3% slower, at 400 x 800 x 266 (243000: the planes under way outgrow the L2s
-   without slab order) 4.61 against 4.09 ms. */
+   8. A batch on variant 32 takes it on vertical columns alone; with nine
+   metric terms its bands stay in their groups, whose sums round differently.
+   Its order has no slabs, so the planes that a z derivative spans have to
+   stay in the L2s; on small planes the last round of blocks, which it fills,
+   weighs more. One launch against two, us per stage, vertical columns / nine
+   terms:
+     200 x 300 x 100 (a plane of 33280)  357, 362 / 388, 396
+     400 x 160 x 80  (38400)             290, 286 / 316, 312
+     260 x 250 x 100 (43392)             343, 349 / 374, 383
+     200 x 400 x 150 (46080)             671, 691 / 732, 760
+     400 x 200 x 80  (51200)             343, 352 / 372, 384
+     260 x 300 x 100 (52992)             417, 406 / 454, 448
+     200 x 460 x 100 (53760)             538, 539 / 585, 593
+     260 x 400 x 80  (72192)             448, 426 / 492, 471
+     200 x 640 x 100 (76800)             728, 732 / 802, 805
+     400 x 800 x 266 (243000)            4610, 4090
+   Three scenarios on 32: 1984, 2073 at 46080, 1225, 1217 at 52992, 1312,
+   1281 at 72192. Below 50000 points it is ahead but for 1.4% at one shape,
+   above it is ahead or behind by up to 5%, in both forms alike. */
 constexpr long kOneLaunchPlane = 48000;
 
 constexpr int kBandSlabBlocks = 192;
@@ -591,10 +604,14 @@ static void box_split(const VolArgs &a, int tw, bool grouped, VolBox &x, VolBand
     r.ox[q] = x0 & ~31;
     r.ntx[q] = (x1 - r.ox[q] + 31) / 32;
     r.nty[q] = (y1 - y0 + 7) / 8;
-    /* a plane of a slab holds at most kBandSlabBlocks blocks, so the seven
-       planes a z derivative reads fit among the ~1500 blocks resident at 6
-       waves per SIMD (a whole plane of the bottom band of a 600 x 1200 grid
-       is 2850 blocks) */
+    /* a plane of a slab holds at most kBandSlabBlocks blocks: the seven
+       planes a z derivative reads should be under way together, and 1280
+       blocks are resident at 5 waves per SIMD (a whole plane of the bottom
+       band of a 600 x 1200 grid is 2850). The time is flat about that size:
+       bands and box per stage with 96, 128, 182, 192, 224, 256 and no limit
+       4165, 4025, 3985, 4050, 3945, 3955, 3965 us at 400 x 800 x 266, 5000,
+       4990, 4960, 4960, 4965, 4940, 4970 at 600 x 1200 x 160, 742, 693, 691,
+       692, 692, 692, 692 at 200 x 400 x 150 */
     r.sy[q] = std::max(1, std::min(r.nty[q], kBandSlabBlocks / r.ntx[q]));
     const long nslab = (r.nty[q] + r.sy[q] - 1) / r.sy[q];
     r.cum[q + 1] = r.cum[q] + (long)r.ntx[q] * r.sy[q] * nslab * (k1 - k0);
@@ -646,8 +663,8 @@ bool volume_one_launch(int variant, const VolArgs &a, int fork) {
    round with box tiles: 55.5 -> 47.6 us per stage at 80 x 120 x 60, 91.6 ->
    82.2 at 96 x 141 x 72, 253 -> 243 at 160 x 240 x 100, 693 -> 674 at 200 x
    400 x 150, six scenarios at 80 x 120 x 60 296 -> 244, twelve at 200 x 400 x
-   150 8.12 -> 7.91 ms. 32-wide tiles unless the box is whole 64-column tiles
-   (its x bounds are multiples of 32; 48.4 against 47.1 us at 80 x 120 x 60). */
+   150 8.12 -> 7.91 ms. 32-wide tiles where 64-wide ones would idle
+   more than a tenth of their lanes (48.4 against 47.1 us at 80 x 120 x 60). */
 template <int ID, int JD, int KD, int TW, bool VC>
 __global__ void __launch_bounds__(256, 5) k_vol_split(VolArgs a, BatArgs b, VolBox x, VolBands r, unsigned per) {
   const int sn = b.act[blockIdx.x / per];
