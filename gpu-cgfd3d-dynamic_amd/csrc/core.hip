@@ -182,8 +182,10 @@ struct cgfd_core {
     if (n == 0) return CGFD_OK;
     void *q = nullptr;
     hipError_t e = hipMalloc(&q, n * sizeof(T));
-    if (e != hipSuccess)
+    if (e != hipSuccess) {
+      (void)hipGetLastError();  /* reported here, not by the next launch's check */
       return cgfd_set_error(CGFD_ERR_NOMEM, "hipMalloc of %zu bytes failed: %s", n * sizeof(T), hipGetErrorString(e));
+    }
     mem.ptrs.push_back(q);
     *p = (T *)q;
     return CGFD_OK;
@@ -972,13 +974,16 @@ int adj_sweep(cgfd_core *c, int scen, const float *residual, const float *residu
   for (int dim = 0; dim < 3; dim++)
     for (int side = 0; side < 2; side++)
       if (c->pml[dim][side].on) npml += 45 * c->pml[dim][side].n;
-  if (!c->adj) {
-    if ((rc = c->alloc(&c->adj, (size_t)4 * lv))) return rc;
-    const size_t nsg = (size_t)9 * sc + (c->isfree ? (size_t)48 * g.siz : 0);  /* S, G; the top-layer sums (AdjTop) */
-    if ((rc = c->alloc(&c->adj_sg, nsg))) return rc;
-    HIPCHK(hipMemset(c->adj_sg, 0, nsg * 4));  /* ghost entries stay zero */
-    if (npml > 0 && (rc = c->alloc(&c->adj_pml, (size_t)npml))) return rc;
+  /* each on its own: a call that ran out of memory leaves the rest to the next one */
+  if (!c->adj && (rc = c->alloc(&c->adj, (size_t)4 * lv))) return rc;
+  const size_t nsg = (size_t)9 * sc + (c->isfree ? (size_t)48 * g.siz : 0);  /* S, G; the top-layer sums (AdjTop) */
+  if (!c->adj_sg) {
+    float *sg = nullptr;
+    if ((rc = c->alloc(&sg, nsg))) return rc;
+    HIPCHK(hipMemset(sg, 0, nsg * 4));  /* ghost entries stay zero */
+    c->adj_sg = sg;
   }
+  if (npml > 0 && !c->adj_pml && (rc = c->alloc(&c->adj_pml, (size_t)npml))) return rc;
   const size_t nadjf = (size_t)c->nfault * kAdjFaultFloats * ss;
   if (c->nfault > 0 && !c->adjf && (rc = c->alloc(&c->adjf, nadjf))) return rc;
   HIPCHK(hipMemsetAsync(c->adj, 0, (size_t)4 * lv * 4, c->st));
